@@ -232,7 +232,7 @@ typedef struct {
 
 /* The quantized matmul on the matrix cores (qgemm.hip): out[t][n] =
  * x[t] . w[n] over f16 weights f16(d * q) and f16 activations, f32
- * accumulation; workgroups of 128 weight rows x TM tokens. */
+ * accumulation; workgroups of 256 weight rows x 128 (MoE: or 64) tokens. */
 typedef struct {
     const uint8_t *w, *w_up;    /* packed weights (gate/up for GLU)          */
     const void *x;              /* [m][ldx] f32 or f16                       */
@@ -257,7 +257,25 @@ typedef struct {
     unsigned long long *status;
     int64_t estride;
     int32_t n_experts, max_pairs, tm, moe_up;
+    int32_t vec, pad_;          /* out rows take four-value stores           */
 } QGemmArgs;
+
+/* The same product for up to 128 activation rows (qgemm_few.hip), and the
+ * rows' rounding to f16 ahead of it (cuca_qgemm_rows_*: x [m][ldx] -> out f16
+ * [m][k], of any alignment). */
+typedef struct {
+    const uint8_t *w, *w_up;    /* packed weights (gate/up for GLU)          */
+    const void *x;              /* [m][ldx]                                  */
+    void *out;                  /* [m][out_ld]                               */
+    int64_t ldx, out_ld, row_bytes;
+    int32_t rows, m, k, nb, ng; /* weight rows; blocks and groups of a row   */
+    int32_t gs;                 /* groups a split (grid y = splits)          */
+    int32_t n_tile, n_ct;       /* weight-tile workgroups, token tiles       */
+    float *part;                /* split sums [splits][g,u][m][rows]         */
+    int32_t gelu, vec;          /* GLU activation; _rows_: 16-byte pieces    */
+    float clamp;
+    int32_t pad_;
+} QGemmFewArgs;
 
 /* The dense f16 path's conversions (qgemm.hip): cuca_qdequant_* (packed w
  * [n][ng][GB], row_bytes each -> out f16 [n][out_ld]) and cuca_cvt_f16_f32

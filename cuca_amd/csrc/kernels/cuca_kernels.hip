@@ -15,5 +15,6 @@
 #include "qmv.hip"
 #include "qmd.hip"
 #include "qgemm.hip"
+#include "qgemm_few.hip"
 #include "gemm16.hip"
 #include "attn_rows.hip"

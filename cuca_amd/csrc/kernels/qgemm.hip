@@ -1,7 +1,7 @@
 // qgemm.hip -- the quantized matmul for many activation rows (prefill, large
-// decode batches) on gfx950's matrix cores: out[t][n] = x[t] . w[n] with
-// the Q4_0 / Q8_0 weights dequantised to f16 and the activations rounded to
-// f16, f32 accumulation (v_mfma_f32_32x32x16_f16).
+// batches) on gfx950's matrix cores: out[t][n] = x[t] . w[n] with the Q4_0 /
+// Q8_0 weights dequantised to f16 and the activations rounded to f16, f32
+// accumulation (v_mfma_f32_16x16x32_f16).  Up to 128 rows: qgemm_few.hip.
 //
 // This is the reference GPU engine's arithmetic class for its dense paths
 // (dense_gemv_kernel / dense_dequant_kernel, moe_kernel.rs:1414-1600: float
@@ -10,106 +10,144 @@
 // each activation f16(x), one rounding each; the error is bounded by
 // (2^-10 + k 2^-24) sum_i |w_i x_i| and the parity tests hold it to that.
 //
-// The weights are read in the packed layout of qmm.hip.  A dot product may
-// sum its terms in any order, so the k index of the matrix-core operands is
-// the packed layout's own order: a lane's 8 f16 of a k-step come from one
-// or two packed dwords (shift, mask, an f16 bias subtracted, the block scale
-// multiplied, two values at a time), and the activations are staged into
-// LDS in the same order.  Slot j of a lane's 8 values is true position
-// base + 16 j:
-//   Q4_0: k-chunk kc = group kc/4, quarter qq = kc%4; k-step s, half h:
-//         lane chunk l = 4 qq + s/2, dword t = 2 h + s%2,
-//         base = 512 g + 128 t + l; dword t of chunk l holds blocks 4t..4t+3
-//         (pair i = nibbles 4i and 16+4i: elements l and l+16 of block 4t+i)
-//   Q8_0: k-chunk kc = group kc/2, half hh = kc%2; k-step s, half h:
-//         lane chunk l = 8 hh + s, dwords 2h and 2h+1, base = 256 g + 128 h + l
-//         (dword t: biased bytes of elements l, l+16 of blocks 2t, 2t+1)
+// Tiling.  A workgroup of 4 waves computes 256 weight rows (the GLU form: 128
+// gate rows and the 128 up rows of the same columns) x NT * 16 tokens; a wave
+// takes 64 rows (32 gate + 32 up) x every token of the tile, 4 x NT tiles of
+// 16 x 16.  Each weight is dequantised once a workgroup, in the registers of
+// the wave that multiplies it, and each activation operand that a wave reads
+// from LDS feeds four products: 32 rows a wave (two products a read) had the
+// LDS busy with the reads all the time.  Two workgroups fit a compute unit,
+// two waves a SIMD, so that one wave's dequantisation (about 14 vector
+// instructions an operand of 8 products) runs under the other's products.
 //
-// Workgroup: 4 waves, 128 weight rows (32 per wave) x TM tokens (TM / 32
-// accumulator tiles per wave); k in chunks of 128 values (8 k-steps).  While
-// a chunk computes, the next chunk's weights are loaded into registers and
-// its activations copied into the other LDS buffer.  The grid is XCD-aware
-// and grouped (qgemm_body).
+// k order.  The weights are read in the packed layout of qmm.hip.  A dot
+// product may sum its terms in any order, so the k index of the operands is
+// the packed layout's own.  k runs in chunks of 128 values, 4 k-steps of 32.
+// A lane (r, u) of a wave loads 16 bytes of row r: lane chunk c0 + u of the
+// group (c0 = the first of the k-chunk's lane chunks), whose dword t holds
+// the pairs of the blocks BPD t ..; the four lanes u of a row then exchange
+// dwords (a 4 x 4 transpose, two permlane swaps of two registers each) so
+// that lane u holds dword u of the chunks c0 .. c0 + 3.  So a lane needs the
+// scales of the blocks BPD u .. only, and one 16-byte load is four k-steps.
+// Slot j of lane u in k-step s is then true position
+//   Q4_0 (512-value groups, a k-chunk = quarter q):
+//        512 g + 128 u + 16 j + 4 q + s
+//   Q8_0 (256-value groups, a k-chunk = half q, two loads a chunk):
+//        256 g + 64 u + 16 (j % 4) + 8 q + 2 s + j / 4
+// and the activations are rewritten in that order once a call
+// (qgemm_prep_body), then copied into LDS directly, a k-chunk ahead.
+//
+// Measured on MI355X, Q4_0, Llama-3-8B shapes at 4096 f16 rows, whole call:
+// gate+up with SwiGLU 853-881 us (1.09-1.13 PFLOP/s, 0.44 of the dense peak;
+// 1260 for the kernel before this one, 128 x 128 tiles of 32 x 32 x 16
+// products), down 468-483 (794), q/o 142-149 (219).  Q8_0: 990-1000, 543-550
+// and 165-167.  What bounds it: the products (two waves a SIMD take turns);
+// Q8_0's loads carry twice the bytes.  Not faster: tiles of 64 tokens in
+// place of a split k where the grid is small (down at 777 rows 136 -> 150
+// us); a second register set for the next chunk's weights spilled.
 #include "common.h"
+#include <type_traits>
 
 typedef _Float16 qg_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 qg_h8 __attribute__((ext_vector_type(8)));
-typedef float qg_acc __attribute__((ext_vector_type(16)));
+typedef float qg_acc __attribute__((ext_vector_type(4)));
 typedef uint32_t qg_u2 __attribute__((ext_vector_type(2)));
 
-#define QG_ROWS 128       // weight rows per workgroup (32 per wave)
-#define QG_KC 128         // values per k-chunk: 8 k-steps of 16
+#define QG_ROWS 256       // weight rows per workgroup (64 per wave)
+#define QG_KC 128         // values per k-chunk: 4 k-steps of 32
 
 template <int FMT> struct QgFmt;
-template <> struct QgFmt<0> { // Q4_0: 4 lane chunks of a 512-value group per k-chunk
-    static constexpr int NW = 4, GB = 288, SCB = 32, KCG = 4;
-};
-template <> struct QgFmt<1> { // Q8_0: 8 lane chunks of a 256-value group per k-chunk
-    static constexpr int NW = 8, GB = 272, SCB = 16, KCG = 2;
-};
+template <> struct QgFmt<0> { static constexpr int GB = 288, SCB = 32, KCG = 4, UNITS = 1; }; // Q4_0
+template <> struct QgFmt<1> { static constexpr int GB = 272, SCB = 16, KCG = 2, UNITS = 2; }; // Q8_0
 
-// The weights a lane needs for one k-chunk: its dword pair of each lane
-// chunk, and the scales of its blocks (Q4_0: blocks 8h..8h+7, Q8_0: 4h..4h+3).
-template <int FMT> struct QgA {
-    qg_u2 w[QgFmt<FMT>::NW];
-    u32x4 sc;
+// A lane's weights of a k-chunk of one 16-row tile (Q4_0 one 16-byte load,
+// Q8_0 two), and its scales there (Q4_0: blocks 4u..4u+3; Q8_0: 2u, 2u+1, in
+// .x).
+template <int FMT> struct QgW {
+    u32x4 c[QgFmt<FMT>::UNITS];
+    qg_u2 s;
 };
-
-template <int FMT>
-__device__ static inline void qg_load_a(const uint8_t *wrow, int kc, int h, QgA<FMT> &o) {
+// tile: a tile's first row, in scalar registers, with the bytes that its rows
+// have (rows past the matrix read as zeros: the buffer's bounds check); off:
+// the lane's row of it plus 16 u.  One vector register addresses all four
+// tiles, where global loads took a pair for each.
+struct QgTile {
+    const uint8_t *p;
+    uint32_t bytes;
+};
+__device__ static inline __amdgpu_buffer_rsrc_t qg_rsrc(const QgTile &t, int64_t at) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(t.p + at), 0, (int)t.bytes, 0x00020000);
+}
+template <int FMT> __device__ static inline u32x4 qg_load(const QgTile &t, int kc, int unit, uint32_t off) {
     using F = QgFmt<FMT>;
-    const int g = kc / F::KCG, part = kc % F::KCG;
-    const uint8_t *grp = wrow + (int64_t)g * F::GB;
-#pragma unroll
-    for (int i = 0; i < F::NW; i++) {
-        const int l = part * F::NW + i;
-        o.w[i] = *reinterpret_cast<const qg_u2 *>(grp + F::SCB + 16 * l + 8 * h);
-    }
-    if (FMT == 0) {
-        o.sc = *reinterpret_cast<const u32x4 *>(grp + 16 * h);
-    } else {
-        const qg_u2 s2 = *reinterpret_cast<const qg_u2 *>(grp + 8 * h);
-        o.sc = u32x4{s2.x, s2.y, 0u, 0u};
-    }
+    const int part = (kc % F::KCG) * F::UNITS + unit; // four 64-byte pieces a group in both formats
+    return __builtin_amdgcn_raw_buffer_load_b128(qg_rsrc(t, (int64_t)(kc / F::KCG) * F::GB + F::SCB + 64 * part), (int)off,
+                                                 0, 0);
+}
+template <int FMT> __device__ static inline qg_u2 qg_load_scales(const QgTile &t, int kc, uint32_t off, int u) {
+    using F = QgFmt<FMT>;
+    const __amdgpu_buffer_rsrc_t grp = qg_rsrc(t, (int64_t)(kc / F::KCG) * F::GB);
+    if (FMT == 0) return __builtin_amdgcn_raw_buffer_load_b64(grp, (int)(off - 8u * (uint32_t)u), 0, 0);
+    return qg_u2{__builtin_amdgcn_raw_buffer_load_b32(grp, (int)(off - 12u * (uint32_t)u), 0, 0), 0u};
 }
 
-__device__ static inline qg_h2 qg_pair(uint32_t u, qg_h2 bias, _Float16 d) {
-    const qg_h2 p = __builtin_bit_cast(qg_h2, u) - bias;
-    return p * qg_h2{d, d};
+// Lane u's register t <-> lane t's register u (u the lane's row of 16).
+__device__ static inline void qg_transpose(u32x4 &v) {
+    const auto p02 = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);
+    const auto p13 = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(p02[0], p13[0], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(p02[1], p13[1], false, false);
+    v = u32x4{a[0], a[1], b[0], b[1]};
 }
-__device__ static inline _Float16 qg_scale(const u32x4 &sc, int i) {
-    const uint32_t w = sc[i >> 1];
+
+// (w & mask) | magic in one instruction (a gfx9 instruction holds one
+// constant outside its registers, so C code for it takes two).
+__device__ static inline uint32_t qg_and_or(uint32_t w, uint32_t mask, uint32_t magic) {
+    uint32_t o;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(o) : "v"(w), "v"(mask), "s"(magic));
+    return o;
+}
+__device__ static inline _Float16 qg_scale(qg_u2 s, int i) {
+    const uint32_t w = i < 2 ? s.x : s.y;
     return __builtin_bit_cast(_Float16, (uint16_t)((i & 1) ? (w >> 16) : (w & 0xffffu)));
 }
 
-// The A operand of k-step s (compile-time s).
-template <int FMT>
-__device__ static inline qg_h8 qg_dequant(const QgA<FMT> &a, int s) {
+// The weight operand of k-step s (compile-time s), from its transposed
+// dwords.  Q4_0: a nibble is placed under an f16 exponent where it stands
+// (bits 0-3 under 1024, bits 4-7 under 64, the upper two after one shift),
+// the bias subtracted (exactly), the block scale multiplied: f16(d * q), one
+// rounding.
+template <int FMT> __device__ static inline qg_h8 qg_dequant(const QgW<FMT> &w, int s) {
     qg_h8 o;
-    if (FMT == 0) {
-        const uint32_t w = a.w[s >> 1][s & 1];
-        const qg_h2 bias = {(_Float16)1032.0f, (_Float16)1032.0f};
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t u = ((w >> (4 * i)) & 0x000f000fu) | 0x64006400u;
-            const qg_h2 p = qg_pair(u, bias, qg_scale(a.sc, (s & 1) * 4 + i));
-            o[2 * i] = p.x;
-            o[2 * i + 1] = p.y;
+    for (int i = 0; i < 4; i++) {
+        uint32_t v;
+        float bias;
+        _Float16 d;
+        if (FMT == 0) {
+            const uint32_t x = i < 2 ? w.c[0][s] : w.c[0][s] >> 8;
+            v = i & 1 ? qg_and_or(x, 0x00f000f0u, 0x54005400u) : qg_and_or(x, 0x000f000fu, 0x64006400u);
+            bias = i & 1 ? 72.0f : 1032.0f;
+            d = qg_scale(w.s, i);
+        } else { // the biased bytes under 0x64
+            v = __builtin_amdgcn_perm(0x64646464u, w.c[(s >> 1) % QgFmt<FMT>::UNITS][2 * (s & 1) + (i >> 1)],
+                                      i & 1 ? 0x04030401u : 0x04020400u);
+            bias = 1152.0f;
+            d = qg_scale(w.s, i & 1);
         }
-    } else {
-        const qg_h2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-#pragma unroll
-        for (int idx = 0; idx < 2; idx++) {
-            const uint32_t w = a.w[s][idx];
-            const qg_h2 p0 = qg_pair(__builtin_amdgcn_perm(0x64646464u, w, 0x04020400u), bias, qg_scale(a.sc, 2 * idx));
-            const qg_h2 p1 = qg_pair(__builtin_amdgcn_perm(0x64646464u, w, 0x04030401u), bias, qg_scale(a.sc, 2 * idx + 1));
-            o[4 * idx + 0] = p0.x;
-            o[4 * idx + 1] = p0.y;
-            o[4 * idx + 2] = p1.x;
-            o[4 * idx + 3] = p1.y;
-        }
+        const qg_h2 p = (__builtin_bit_cast(qg_h2, v) - qg_h2{(_Float16)bias, (_Float16)bias}) * qg_h2{d, d};
+        o[2 * i] = p.x;
+        o[2 * i + 1] = p.y;
     }
     return o;
+}
+
+// True position of slot 0 of unit v = 4 s + u (k-step s, lane u) of k-chunk
+// kc, and of slot j.
+template <int FMT> __device__ static inline int qg_slot(int kc, int v, int j) {
+    const int s = v >> 2, u = v & 3;
+    if (FMT == 0) return 512 * (kc >> 2) + 128 * u + 16 * j + 4 * (kc & 3) + s;
+    return 256 * (kc >> 1) + 64 * u + 16 * (j & 3) + 8 * (kc & 1) + 2 * s + (j >> 2);
 }
 
 __device__ static inline void qgemm_load8f(const float *p, float (&v)[8]) {
@@ -122,91 +160,36 @@ __device__ static inline void qgemm_load8f(const float *p, float (&v)[8]) {
 // The activations rewritten once per call, before the matmul: f16, in the
 // slot order of the format (xp [n_ct * TM][kp], kp = 128 per k-chunk; zero
 // past k and in the rows past m, up to the whole tile).  One thread per unit
-// (token, k-chunk, k-step s, half h) of 8 values: the values at true
-// positions base + 16 j.
+// (token, k-chunk, v = 4 k-step + lane u) of 8 values.
 template <typename T, int FMT> __device__ static inline void qgemm_prep_body(const QGemmArgs &a) {
-    using F = QgFmt<FMT>;
     const int64_t u = (int64_t)blockIdx.x * CUCA_BLOCK + threadIdx.x;
     const int64_t per_row = (int64_t)a.nkc * 16;
     if (u >= (int64_t)a.mp * per_row) return;
     const int tok = (int)(u / per_row), rem = (int)(u - (int64_t)tok * per_row);
-    const int kc = rem >> 4, v = rem & 15, s = v >> 1, h = v & 1;
-    const int g = kc / F::KCG, part = kc % F::KCG;
-    int base;
-    if (FMT == 0) base = 512 * g + 128 * (2 * h + (s & 1)) + 4 * part + (s >> 1);
-    else base = 256 * g + 128 * h + 8 * part + s;
+    const int kc = rem >> 4, v = rem & 15;
     const T *row = reinterpret_cast<const T *>(a.x) + (int64_t)(tok < a.m ? tok : 0) * a.ldx;
     qg_h8 o;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        const int k = base + 16 * j;
+        const int k = qg_slot<FMT>(kc, v, j);
         o[j] = tok < a.m && k < a.k ? (_Float16)(float)row[k] : (_Float16)0.0f;
     }
-    *reinterpret_cast<qg_h8 *>(a.xp + (int64_t)tok * a.kp + (int64_t)kc * QG_KC + 8 * (2 * s + h)) = o; // xp: f16 bits
-}
-
-// The activations of one k-chunk, TM tokens x 128 f16, copied from the
-// workspace straight into LDS (global_load_lds_dwordx4: lane L of a wave
-// writes 16 bytes at the wave's LDS address + 16 L).  A row is 256 bytes,
-// unpadded; its 16-byte unit v sits at position v ^ (row % 16), so that the
-// B-operand reads of 16 rows at one unit fall in different banks.  Wave w's
-// copy it fills rows 16 it + 4 w .. + 3.
-// The lane's part of the source offset, lane_off = (lane / 16) kp + 8 v, is
-// the same for every copy (row % 16 = (4 w + lane / 16) % 16).
-template <int TM>
-__device__ static inline void qg_copy_x(const QGemmArgs &a, int tok0, int kc, int wave, int lane_off,
-                                        _Float16 (*xs)[QG_KC]) {
-#pragma unroll
-    for (int it = 0; it < TM / 16; it++) {
-        const int c0 = 16 * it + 4 * wave; // wave-uniform
-        const uint16_t *src = a.xp + ((int64_t)(tok0 + c0) * a.kp + (int64_t)kc * QG_KC);
-        __builtin_amdgcn_global_load_lds(src + lane_off, &xs[c0][0], 16, 0, 0);
-    }
-}
-
-// One k-chunk: the MFMAs over xc, while the next chunk's activations are
-// copied into xn and its weights loaded into ng / nu.
-template <int FMT, int TM, bool GLU>
-__device__ static inline void qg_chunk(const QGemmArgs &a, const uint8_t *wg, const uint8_t *wu, int tok0, int kc,
-                                       bool next, int wave, int lane, int lane_off, _Float16 (*xc)[QG_KC],
-                                       _Float16 (*xn)[QG_KC],
-                                       QgA<FMT> &ag, QgA<FMT> &au, qg_acc *acc, qg_acc *accu) {
-    constexpr int NT = TM / 32;
-    const int r = lane & 31, h = lane >> 5;
-    QgA<FMT> ng, nu;
-    if (next) {
-        qg_load_a<FMT>(wg, kc + 1, h, ng);
-        if (GLU) qg_load_a<FMT>(wu, kc + 1, h, nu);
-        qg_copy_x<TM>(a, tok0, kc + 1, wave, lane_off, xn);
-    }
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const qg_h8 av = qg_dequant<FMT>(ag, s);
-        qg_h8 uv;
-        if (GLU) uv = qg_dequant<FMT>(au, s);
-        const int pos = 8 * ((2 * s + h) ^ (r & 15));
-#pragma unroll
-        for (int i = 0; i < NT; i++) {
-            const qg_h8 bv = *reinterpret_cast<const qg_h8 *>(&xc[i * 32 + r][pos]);
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc[i], 0, 0, 0);
-            if (GLU) accu[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(uv, bv, accu[i], 0, 0, 0);
-        }
-    }
-    __builtin_amdgcn_s_waitcnt(0); // the copies into xn have landed
-    __syncthreads();
-    if (next) {
-        ag = ng;
-        if (GLU) au = nu;
-    }
+    *reinterpret_cast<qg_h8 *>(a.xp + (int64_t)tok * a.kp + (int64_t)kc * QG_KC + 8 * v) = o; // xp: f16 bits
 }
 
 // SPLIT: workgroup (tile, split) takes k-chunks [split * kcs, ...) and
 // writes its f32 sums to the partial rows of the workspace (qgemm_reduce
 // adds the splits in order and applies the epilogue); otherwise the
 // epilogue is applied here.
-template <typename T, int FMT, int TM, bool GLU, int ACT, bool SPLIT, int MOE = 0>
+template <typename T, int FMT, int NT, bool GLU, int ACT, bool SPLIT, int MOE = 0>
 __device__ static inline void qgemm_body(const QGemmArgs &a) {
-    constexpr int NT = TM / 32;
+    using F = QgFmt<FMT>;
+    constexpr int TM = NT * 16;
+    constexpr int COLS = GLU ? QG_ROWS / 2 : QG_ROWS; // output columns of a workgroup
+    // two buffers of a k-chunk's activations: rows of 256 bytes, 16-byte unit
+    // v of row R at unit v ^ (R & 7), so that the reads of 8 rows at one unit
+    // fall in different banks
+    __shared__ __attribute__((aligned(16))) _Float16 xs[2 * TM * QG_KC];
     const int split = SPLIT ? (int)blockIdx.y : 0;
     // XCD x (workgroups x, x + 8, ...) takes row tiles x, x + 8, ... in
     // groups of 8; a group's workgroups take its row tiles in turn, token
@@ -233,110 +216,178 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     if (kc0 >= kc1) return;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 31, h = lane >> 5;
-    const int row = rt * QG_ROWS + wave * 32 + r;
+    const int r = lane & 15, u = lane >> 4;
     const int tok0 = ct * TM;
-    const int64_t roff = (int64_t)(row < a.rows ? row : 0) * a.row_bytes + (MOE ? (int64_t)ex * a.estride : 0);
-    const uint8_t *wg = a.w + roff;
-    const uint8_t *wu = GLU ? a.w_up + roff : nullptr;
-
-    qg_acc acc[NT], accu[NT];
+    const int n0 = rt * COLS + wave * (COLS / 4); // the wave's first output column
+    // the wave's 16-row tiles (GLU: gate, gate, up, up of the same columns)
+    QgTile tile[4];
 #pragma unroll
-    for (int i = 0; i < NT; i++) {
-        acc[i] = qg_acc{};
-        accu[i] = qg_acc{};
+    for (int i = 0; i < 4; i++) {
+        const int r0 = n0 + 16 * (GLU ? i & 1 : i); // uniform
+        const int left = max(0, min(16, a.rows - r0));
+        const uint64_t p = (uint64_t)(uintptr_t)(GLU && i >= 2 ? a.w_up : a.w) + (uint64_t)((int64_t)r0 * a.row_bytes) +
+                           (MOE ? (uint64_t)((int64_t)ex * a.estride) : 0);
+        const uint64_t ps = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32) |
+                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p);
+        tile[i].p = reinterpret_cast<const uint8_t *>((uintptr_t)ps);
+        const uint64_t bytes = (uint64_t)left * (uint64_t)a.row_bytes; // (16 rows of k = 2^28 pass 32 bits; 15 do not)
+        tile[i].bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(bytes < 0xffffffffull ? bytes : 0xffffffffull));
     }
-    // two LDS buffers, separate objects so that the compiler sees the copy
-    // into one and the reads of the other do not overlap
-    __shared__ __attribute__((aligned(16))) _Float16 xs0[TM][QG_KC];
-    __shared__ __attribute__((aligned(16))) _Float16 xs1[TM][QG_KC];
-    QgA<FMT> ag, au;
-    qg_load_a<FMT>(wg, kc0, h, ag);
-    if (GLU) qg_load_a<FMT>(wu, kc0, h, au);
-    const int lane_off = (lane >> 4) * (int)a.kp + 8 * ((lane & 15) ^ ((4 * wave + (lane >> 4)) & 15));
-    qg_copy_x<TM>(a, tok0, kc0, wave, lane_off, xs0);
-    __builtin_amdgcn_s_waitcnt(0);
+    const uint32_t woff = (uint32_t)r * (uint32_t)a.row_bytes + 16u * (uint32_t)u;
+    // The copies: wave w fills LDS rows w TM / 4 .., four rows of 256 bytes an
+    // instruction (lane L: row L / 16 of them, unit L % 16, from source unit
+    // (L % 16) ^ (row & 7)).  Issued from inline assembly with the waits
+    // written out: the compiler cannot tell the two buffers apart behind an
+    // LDS DMA and would wait for the copies before any LDS read.
+    uint32_t off[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+        off[i] = 2u * ((uint32_t)(lane >> 4) * (uint32_t)a.kp + 8u * (uint32_t)((lane & 15) ^ ((4 * i + (lane >> 4)) & 7)));
+    const uint64_t xv = (uint64_t)(uintptr_t)a.xp + 2 * (uint64_t)((int64_t)(tok0 + wave * (TM / 4)) * a.kp);
+    const uint64_t xb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(xv >> 32)) << 32) |
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)xv);
+    const uint64_t x4 = 8 * (uint64_t)a.kp; // bytes of four rows
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    auto copy = [&](int kc, int buf) {
+#pragma unroll
+        for (int i = 0; i < TM / 16; i++) {
+            const uint64_t src = xb + i * x4 + (uint64_t)kc * (2 * QG_KC);
+            const uint32_t dst = (uint32_t)(uintptr_t)&xs[(buf * TM + wave * (TM / 4) + 4 * i) * QG_KC];
+            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off[i & 1]), "s"(src), "s"(dst)
+                         : "memory", "m0");
+        }
+    };
+#pragma clang diagnostic pop
+    qg_acc acc[4][NT];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = qg_acc{};
+    // weights: a tile's next chunk is requested into its own registers, right
+    // after the last operand made from them (a second register set, a chunk
+    // ahead, spilled)
+    QgW<FMT> wv[4];
+    auto load = [&](int kc, int i, int unit) {
+        const int c = kc < kc1 ? kc : kc1 - 1; // (the last again past the end, unused)
+        wv[i].c[unit] = qg_load<FMT>(tile[i], c, unit, woff);
+        if (unit == F::UNITS - 1) wv[i].s = qg_load_scales<FMT>(tile[i], c, woff, u);
+    };
+    // unit (4 s + u) ^ (r & 7) of row 16 j + r: the k-step's part is s ^ (r >>
+    // 2 & 1), so two addresses and constant offsets serve every read
+    const _Float16 *xe = xs + r * QG_KC + 8 * (u ^ (r & 3)) + 32 * ((r >> 2) & 1), *xo = xe + (r & 4 ? -32 : 32);
+    qg_h8 b[NT];
+    auto read = [&](int buf, int s, int j) {
+        b[j] = *reinterpret_cast<const qg_h8 *>((s & 1 ? xo : xe) + (buf * TM + 16 * j) * QG_KC + 64 * (s >> 1));
+    };
+    constexpr int STEPS = 4 / F::UNITS; // k-steps a load
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int q = 0; q < F::UNITS; q++) load(kc0, i, q);
+    copy(kc0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    for (int kc = kc0; kc < kc1; kc += 2) {
-        qg_chunk<FMT, TM, GLU>(a, wg, wu, tok0, kc, kc + 1 < kc1, wave, lane, lane_off, xs0, xs1, ag, au, acc, accu);
-        if (kc + 1 < kc1)
-            qg_chunk<FMT, TM, GLU>(a, wg, wu, tok0, kc + 1, kc + 2 < kc1, wave, lane, lane_off, xs1, xs0, ag, au, acc, accu);
-    }
-    // accumulator q of lane (r, h): weight row 8 (q / 4) + 4 h + q % 4, token r.
-    // The empty asm keeps a tile in the accumulator registers until its turn
-    // (after the previous tile's stores): copied out all at once, the tiles
-    // would set the kernel's register count.
-    if (SPLIT) {
-        // partial rows: [split][gate, up][m][rows] f32
+    // (the buffer is a run-time value: unrolled by two with constant buffers,
+    // the Q4_0 kernels spilled)
+    for (int kc = kc0, buf = 0; kc < kc1; kc++, buf ^= 1) {
+        if (kc + 1 < kc1) copy(kc + 1, buf ^ 1);
 #pragma unroll
-        for (int i = 0; i < NT; i++) {
-            asm volatile("" : "+a"(acc[i]));
-            if (GLU) asm volatile("" : "+a"(accu[i]));
-            const int tok = tok0 + i * 32 + r;
-            if (tok >= a.m) continue;
-            float *pg = a.part + ((int64_t)split * (GLU ? 2 : 1) * a.m + tok) * a.rows;
-            float *pu = a.part + ((int64_t)(split * 2 + 1) * a.m + tok) * a.rows;
+        for (int j = 0; j < NT; j++) read(buf, 0, j);
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int n = rt * QG_ROWS + wave * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-                if (n >= a.rows) continue;
-                pg[n] = acc[i][q];
-                if (GLU) pu[n] = accu[i][q];
+        for (int s = 0; s < 4; s++) {
+            if (s % STEPS == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) qg_transpose(wv[i].c[s / STEPS]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const qg_h8 av = qg_dequant<FMT>(wv[i], s);
+                if (s % STEPS == STEPS - 1) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(kc + 1, i, s / STEPS);
+                }
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[j], acc[i][j], 0, 0, 0);
+                    if (i == 3 && s < 3) read(buf, s + 1, j); // the next k-step's operand
+                }
+                // an operand is dequantised no further ahead (the kernels spill otherwise)
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        return;
+        // The next chunk's copies have landed, and every wave is done with
+        // this buffer.  Of a wave's loads only the weight loads above come
+        // after its copies (a load does not pass an asm with a memory
+        // clobber), so that many may stay in flight.
+        if constexpr (F::UNITS == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        __syncthreads();
     }
-    if (MOE) {
-        // pair p0 + local of the tile: up, act(g) * u into hidden row p; down,
-        // the f32 product times the pair's routing weight into scratch row p
+    // accumulator e of lane (r, u) in tile (i, j): weight row 16 i + 4 u + e
+    // of the wave's, token 16 j + r.  The empty asm keeps a tile where it is
+    // until its turn (copied out all at once, the tiles would set the
+    // kernel's register count).
+    constexpr int NI = GLU && !SPLIT ? 2 : 4;
 #pragma unroll
-        for (int i = 0; i < NT; i++) {
-            asm volatile("" : "+a"(acc[i]));
-            if (GLU) asm volatile("" : "+a"(accu[i]));
-            const int local = i * 32 + r;
-            if (local >= np) continue;
-            const int64_t p = p0 + local;
-            const float pw = MOE == 2 ? a.pair_weight[p] : 1.0f;
+    for (int j = 0; j < NT; j++) {
+        const int local = 16 * j + r;
+        const int tok = tok0 + local;
+        const bool live = MOE ? local < np : tok < a.m;
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int n = rt * QG_ROWS + wave * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-                if (n >= a.rows) continue;
-                float o = acc[i][q];
+        for (int i = 0; i < NI; i++) {
+            asm volatile("" : "+v"(acc[i][j]));
+            if (GLU && !SPLIT) asm volatile("" : "+v"(acc[i + 2][j]));
+            if (!live) continue;
+            const int c = n0 + 16 * (GLU ? i & 1 : i) + 4 * u;
+            if (SPLIT) { // partial rows: [split][gate, up][m][rows] f32
+                const int64_t mat = GLU ? (int64_t)split * 2 + (i >> 1) : split;
+                float *o = a.part + (mat * a.m + tok) * a.rows + c;
+                if ((a.rows & 3) == 0 && c < a.rows) {
+                    *reinterpret_cast<f32x4 *>(o) = acc[i][j];
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (c + e < a.rows) o[e] = acc[i][j][e];
+                }
+                continue;
+            }
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = acc[i][j][e];
                 if (GLU) {
-                    float gg = o, u = accu[i][q];
+                    float gg = v[e], uu = acc[(i + 2) & 3][j][e];
                     if (a.clamp > 0.0f) { // Glu::apply's clamp (cpu.rs:364-368)
                         gg = fminf(gg, a.clamp);
-                        u = fminf(fmaxf(u, -a.clamp), a.clamp);
+                        uu = fminf(fmaxf(uu, -a.clamp), a.clamp);
                     }
-                    o = (ACT == 0 ? act_silu(gg) : act_gelu_tanh(gg)) * u;
+                    v[e] = (ACT == 0 ? act_silu(gg) : act_gelu_tanh(gg)) * uu;
                 }
-                if (MOE == 2) reinterpret_cast<float *>(a.out)[p * a.out_ld + n] = o * pw;
-                else reinterpret_cast<T *>(a.out)[p * a.out_ld + n] = to_stored<T>(o);
             }
-        }
-        return;
-    }
+            // MoE: pair p0 + local; down, the f32 product times the pair's
+            // routing weight into the scratch row
+            const int64_t row = MOE ? p0 + local : tok;
+            if (MOE == 2) {
+                const float pw = a.pair_weight[row];
 #pragma unroll
-    for (int i = 0; i < NT; i++) {
-        asm volatile("" : "+a"(acc[i]));
-        if (GLU) asm volatile("" : "+a"(accu[i]));
-        const int tok = tok0 + i * 32 + r;
-        if (tok >= a.m) continue;
-        T *orow = reinterpret_cast<T *>(a.out) + (int64_t)tok * a.out_ld;
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const int n = rt * QG_ROWS + wave * 32 + 8 * (q >> 2) + 4 * h + (q & 3);
-            if (n >= a.rows) continue;
-            float o = acc[i][q];
-            if (GLU) {
-                float g = o, u = accu[i][q];
-                if (a.clamp > 0.0f) { // Glu::apply's clamp (cpu.rs:364-368)
-                    g = fminf(g, a.clamp);
-                    u = fminf(fmaxf(u, -a.clamp), a.clamp);
+                for (int e = 0; e < 4; e++) v[e] *= pw;
+            }
+            typedef typename std::conditional<MOE == 2, float, T>::type O;
+            O *o = reinterpret_cast<O *>(a.out) + row * a.out_ld + c;
+            if (a.vec && c + 3 < a.rows) {
+                if (sizeof(O) == 4) {
+                    *reinterpret_cast<f32x4 *>(o) = f32x4{v[0], v[1], v[2], v[3]};
+                } else {
+                    typedef _Float16 qg_h4 __attribute__((ext_vector_type(4)));
+                    *reinterpret_cast<qg_h4 *>(o) = qg_h4{to_stored<_Float16>(v[0]), to_stored<_Float16>(v[1]),
+                                                         to_stored<_Float16>(v[2]), to_stored<_Float16>(v[3])};
                 }
-                o = (ACT == 0 ? act_silu(g) : act_gelu_tanh(g)) * u;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (c + e < a.rows) o[e] = to_stored<O>(v[e]);
             }
-            orow[n] = to_stored<T>(o);
         }
     }
 }
@@ -415,18 +466,13 @@ __device__ static inline void qgemm_moe_plan_body(const QGemmArgs &a) {
 // outside [0, m) gives a zero row, reported), down row p.  Tiles past the
 // last are not written (the GEMM skips them).
 template <typename T, int FMT> __device__ static inline void qgemm_moe_prep_body(const QGemmArgs &a) {
-    using F = QgFmt<FMT>;
     const int64_t u = (int64_t)blockIdx.x * CUCA_BLOCK + threadIdx.x;
     const int64_t per_row = (int64_t)a.nkc * 16;
     if (u >= (int64_t)a.mp * per_row) return;
     const int prow = (int)(u / per_row), rem = (int)(u - (int64_t)prow * per_row);
     const int ct = prow / a.tm, i = prow - ct * a.tm;
     if (a.tile_e[ct] < 0) return;
-    const int kc = rem >> 4, v = rem & 15, s = v >> 1, h = v & 1;
-    const int g = kc / F::KCG, part = kc % F::KCG;
-    int base;
-    if (FMT == 0) base = 512 * g + 128 * (2 * h + (s & 1)) + 4 * part + (s >> 1);
-    else base = 256 * g + 128 * h + 8 * part + s;
+    const int kc = rem >> 4, v = rem & 15;
     bool valid = i < a.tile_n[ct];
     int64_t src = 0;
     if (valid) {
@@ -447,34 +493,35 @@ template <typename T, int FMT> __device__ static inline void qgemm_moe_prep_body
     qg_h8 o;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        const int k = base + 16 * j;
+        const int k = qg_slot<FMT>(kc, v, j);
         o[j] = valid && k < a.k ? (_Float16)(float)row[k] : (_Float16)0.0f;
     }
-    *reinterpret_cast<qg_h8 *>(a.xp + (int64_t)prow * a.kp + (int64_t)kc * QG_KC + 8 * (2 * s + h)) = o;
+    *reinterpret_cast<qg_h8 *>(a.xp + (int64_t)prow * a.kp + (int64_t)kc * QG_KC + 8 * v) = o;
 }
 
 #define CUCA_QGEMM(NAME, BODY, ...)                                                        \
     extern "C" __global__ __launch_bounds__(256) void NAME(QGemmArgs a) { BODY<__VA_ARGS__>(a); }
-#define CUCA_QGEMM_TM(TN, T, FN, FMT, TM)                                                  \
-    CUCA_QGEMM(cuca_qgemm_##TN##_##FN##_t##TM, qgemm_body, T, FMT, TM, false, 0, false)    \
-    CUCA_QGEMM(cuca_qgemm_glu_##TN##_##FN##_silu_t##TM, qgemm_body, T, FMT, TM, true, 0, false) \
-    CUCA_QGEMM(cuca_qgemm_glu_##TN##_##FN##_gelu_t##TM, qgemm_body, T, FMT, TM, true, 1, false) \
-    CUCA_QGEMM(cuca_qgemm_##TN##_##FN##_t##TM##_split, qgemm_body, T, FMT, TM, false, 0, true) \
-    CUCA_QGEMM(cuca_qgemm_glu_##TN##_##FN##_t##TM##_split, qgemm_body, T, FMT, TM, true, 0, true)
+// two workgroups a compute unit: at most 256 registers
+#define CUCA_QGEMM_TILE(NAME, ...)                                                         \
+    extern "C" __global__ __launch_bounds__(256, 2) void NAME(QGemmArgs a) { qgemm_body<__VA_ARGS__>(a); }
 #define CUCA_QGEMM_SET(TN, T, FN, FMT)                                                     \
     CUCA_QGEMM(cuca_qgemm_prep_##TN##_##FN, qgemm_prep_body, T, FMT)                        \
-    CUCA_QGEMM_TM(TN, T, FN, FMT, 32)                                                      \
-    CUCA_QGEMM_TM(TN, T, FN, FMT, 64)                                                      \
-    CUCA_QGEMM_TM(TN, T, FN, FMT, 128)
+    CUCA_QGEMM_TILE(cuca_qgemm_##TN##_##FN, T, FMT, 8, false, 0, false)                    \
+    CUCA_QGEMM_TILE(cuca_qgemm_glu_##TN##_##FN##_silu, T, FMT, 8, true, 0, false)          \
+    CUCA_QGEMM_TILE(cuca_qgemm_glu_##TN##_##FN##_gelu, T, FMT, 8, true, 1, false)
 CUCA_QGEMM_SET(f32, float, q4_0, 0)
 CUCA_QGEMM_SET(f32, float, q8_0, 1)
 CUCA_QGEMM_SET(f16, _Float16, q4_0, 0)
 CUCA_QGEMM_SET(f16, _Float16, q8_0, 1)
+CUCA_QGEMM_TILE(cuca_qgemm_q4_0_split, float, 0, 8, false, 0, true)
+CUCA_QGEMM_TILE(cuca_qgemm_q8_0_split, float, 1, 8, false, 0, true)
+CUCA_QGEMM_TILE(cuca_qgemm_glu_q4_0_split, float, 0, 8, true, 0, true)
+CUCA_QGEMM_TILE(cuca_qgemm_glu_q8_0_split, float, 1, 8, true, 0, true)
 extern "C" __global__ __launch_bounds__(256) void cuca_qgemm_moe_plan(QGemmArgs a) { qgemm_moe_plan_body(a); }
 #define CUCA_QGEMM_MOE_TM(TN, T, FN, FMT, TM)                                              \
-    CUCA_QGEMM(cuca_qgemm_moe_up_##TN##_##FN##_silu_t##TM, qgemm_body, T, FMT, TM, true, 0, false, 1) \
-    CUCA_QGEMM(cuca_qgemm_moe_up_##TN##_##FN##_gelu_t##TM, qgemm_body, T, FMT, TM, true, 1, false, 1) \
-    CUCA_QGEMM(cuca_qgemm_moe_down_##TN##_##FN##_t##TM, qgemm_body, T, FMT, TM, false, 0, false, 2)
+    CUCA_QGEMM_TILE(cuca_qgemm_moe_up_##TN##_##FN##_silu_t##TM, T, FMT, TM / 16, true, 0, false, 1) \
+    CUCA_QGEMM_TILE(cuca_qgemm_moe_up_##TN##_##FN##_gelu_t##TM, T, FMT, TM / 16, true, 1, false, 1) \
+    CUCA_QGEMM_TILE(cuca_qgemm_moe_down_##TN##_##FN##_t##TM, T, FMT, TM / 16, false, 0, false, 2)
 #define CUCA_QGEMM_MOE_SET(TN, T, FN, FMT)                                                 \
     CUCA_QGEMM(cuca_qgemm_moe_prep_##TN##_##FN, qgemm_moe_prep_body, T, FMT)               \
     CUCA_QGEMM_MOE_TM(TN, T, FN, FMT, 64)                                                  \

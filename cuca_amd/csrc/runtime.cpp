@@ -2208,6 +2208,93 @@ cuca_status cuca_hip_qgemm_workspace(uint32_t ggml_type, int64_t n, int64_t k, i
     return CUCA_OK;
 }
 
+// Up to kQgFewRows activation rows: the kernels of qgemm_few.hip, one launch
+// (two where the rows are rounded to f16 first).
+constexpr int64_t kQgFewRows = 128;
+
+static cuca_status qgemm_few(cuca_hip_ctx *ctx, const void *w, const void *w_up, bool q8, int64_t k, int64_t row_bytes,
+                             int group, const void *x, int64_t ldx, int64_t m, int64_t rows, int glu, float clamp,
+                             void *ws, float *part, size_t part_bytes, void *out, int64_t out_ld,
+                             cuca_dtype dtype) {
+    QGemmFewArgs a{};
+    a.w = static_cast<const uint8_t *>(w);
+    a.w_up = static_cast<const uint8_t *>(w_up);
+    a.row_bytes = row_bytes;
+    a.rows = (int32_t)rows;
+    a.m = (int32_t)m;
+    a.k = (int32_t)k;
+    a.nb = (int32_t)(k / 32);
+    a.ng = (a.nb + group - 1) / group;
+    a.gelu = glu == 2;
+    a.clamp = clamp > 0.0f ? clamp : 0.0f;
+    // The kernels read the caller's rows in 16-byte (f32) or 8-byte (f16)
+    // pieces.  Other rows, rows that the output overlaps (workgroups write it
+    // while others still read), and more than 32 f32 rows (which every weight
+    // tile would read at twice the bytes: gate+up of the 8B shapes at 64 rows)
+    // are rounded to f16 into the workspace first.
+    bool half = dtype == CUCA_F16;
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), oa = reinterpret_cast<uintptr_t>(out), es = half ? 2 : 4;
+    const bool aligned = xa % (4 * es) == 0 && ldx % 4 == 0;
+    const bool apart = xa + ((m - 1) * ldx + k) * es <= oa || oa + ((m - 1) * out_ld + rows) * es <= xa;
+    if (!aligned || !apart || (!half && m > 32)) {
+        a.x = x;
+        a.ldx = ldx;
+        a.out = ws;
+        a.vec = al16(x) && ldx % (half ? 8 : 4) == 0;
+        const cuca_status st = launch(ctx, half ? cuca_qgemm_rows_f16 : cuca_qgemm_rows_f32,
+                                      div_up(m * (k / 8), CUCA_BLOCK_THREADS), CUCA_BLOCK_THREADS, 0, a);
+        if (st != CUCA_OK) return st;
+        half = true;
+        a.x = ws;
+        a.ldx = k;
+    } else {
+        a.x = x;
+        a.ldx = ldx;
+    }
+    a.out = out;
+    a.out_ld = out_ld;
+    const int ni = m <= 16 ? 0 : m <= 32 ? 1 : 2; // 16, 32, 64 tokens a tile
+    a.n_ct = (int32_t)((m + (16 << ni) - 1) / (16 << ni));
+    const int64_t wide = glu ? 64 : 128; // output columns a workgroup
+    a.n_tile = (int32_t)((rows + wide - 1) / wide);
+    // split k where the tiles leave compute units idle
+    const int64_t tiles = (int64_t)a.n_tile * a.n_ct;
+    int64_t splits = std::min<int64_t>(kQgMaxSplits, std::max<int64_t>(1, ctx->cu_count / tiles));
+    splits = std::min<int64_t>(splits, (int64_t)(part_bytes / ((size_t)(glu ? 2 : 1) * (size_t)m * (size_t)rows * 4)));
+    splits = std::max<int64_t>(1, std::min<int64_t>(splits, a.ng));
+    a.gs = (int32_t)((a.ng + splits - 1) / splits);
+    splits = (a.ng + a.gs - 1) / a.gs;
+    a.part = part;
+    // [activations f32, f16 -> f32, f16 -> f16][glu][format][tokens a tile]
+    static const Kernel table_k[3][2][2][3] = {
+        {{{cuca_qgemm_few_f32_f32_q4_0_n1, cuca_qgemm_few_f32_f32_q4_0_n2, cuca_qgemm_few_f32_f32_q4_0_n2},
+          {cuca_qgemm_few_f32_f32_q8_0_n1, cuca_qgemm_few_f32_f32_q8_0_n2, cuca_qgemm_few_f32_f32_q8_0_n2}},
+         {{cuca_qgemm_few_glu_f32_f32_q4_0_n1, cuca_qgemm_few_glu_f32_f32_q4_0_n2, cuca_qgemm_few_glu_f32_f32_q4_0_n2},
+          {cuca_qgemm_few_glu_f32_f32_q8_0_n1, cuca_qgemm_few_glu_f32_f32_q8_0_n2, cuca_qgemm_few_glu_f32_f32_q8_0_n2}}},
+        {{{cuca_qgemm_few_f16_f32_q4_0_n1, cuca_qgemm_few_f16_f32_q4_0_n2, cuca_qgemm_few_f16_f32_q4_0_n4},
+          {cuca_qgemm_few_f16_f32_q8_0_n1, cuca_qgemm_few_f16_f32_q8_0_n2, cuca_qgemm_few_f16_f32_q8_0_n4}},
+         {{cuca_qgemm_few_glu_f16_f32_q4_0_n1, cuca_qgemm_few_glu_f16_f32_q4_0_n2, cuca_qgemm_few_glu_f16_f32_q4_0_n4},
+          {cuca_qgemm_few_glu_f16_f32_q8_0_n1, cuca_qgemm_few_glu_f16_f32_q8_0_n2, cuca_qgemm_few_glu_f16_f32_q8_0_n4}}},
+        {{{cuca_qgemm_few_f16_f16_q4_0_n1, cuca_qgemm_few_f16_f16_q4_0_n2, cuca_qgemm_few_f16_f16_q4_0_n4},
+          {cuca_qgemm_few_f16_f16_q8_0_n1, cuca_qgemm_few_f16_f16_q8_0_n2, cuca_qgemm_few_f16_f16_q8_0_n4}},
+         {{cuca_qgemm_few_glu_f16_f16_q4_0_n1, cuca_qgemm_few_glu_f16_f16_q4_0_n2, cuca_qgemm_few_glu_f16_f16_q4_0_n4},
+          {cuca_qgemm_few_glu_f16_f16_q8_0_n1, cuca_qgemm_few_glu_f16_f16_q8_0_n2, cuca_qgemm_few_glu_f16_f16_q8_0_n4}}}};
+    const Kernel kern = table_k[dtype == CUCA_F16 ? 2 : half ? 1 : 0][glu != 0][q8][ni];
+    const cuca_status st = launch2(ctx, kern, (unsigned)(((int64_t)a.n_tile + 7) / 8 * 8 * a.n_ct), (unsigned)splits, 512, 0, a);
+    if (st != CUCA_OK || splits == 1) return st;
+    QGemmArgs r{};
+    r.part = part;
+    r.out = out;
+    r.out_ld = out_ld;
+    r.rows = a.rows;
+    r.m = a.m;
+    r.splits = (int32_t)splits;
+    r.clamp = a.clamp;
+    static const Kernel red_k[2][3] = {{cuca_qgemm_reduce_f32, cuca_qgemm_reduce_glu_f32_silu, cuca_qgemm_reduce_glu_f32_gelu},
+                                       {cuca_qgemm_reduce_f16, cuca_qgemm_reduce_glu_f16_silu, cuca_qgemm_reduce_glu_f16_gelu}};
+    return launch(ctx, red_k[dtype == CUCA_F16][glu], div_up(m * rows, CUCA_BLOCK_THREADS), CUCA_BLOCK_THREADS, 0, r);
+}
+
 // glu: 0 plain, 1 SiLU, 2 GELU-tanh.
 static cuca_status qgemm_common(cuca_hip_ctx *ctx, const void *w, const void *w_up, uint32_t ggml_type, int64_t n,
                                 int64_t k, const void *x, int64_t ldx, int64_t m, int64_t rows, int glu, float clamp,
@@ -2237,18 +2324,25 @@ static cuca_status qgemm_common(cuca_hip_ctx *ctx, const void *w, const void *w_
     if (ws_bytes < xp_bytes)
         return fail(ctx, CUCA_INVALID_ARG, "qgemm: workspace of %zu bytes, %zu needed (cuca_hip_qgemm_workspace)",
                     ws_bytes, xp_bytes);
-    const int tm = qgemm_tm(m);
-    const int ti = tm == 32 ? 0 : tm == 64 ? 1 : 2;
-    const int64_t n_rt = (rows + 127) / 128, n_ct = qgemm_mp(m) / tm;
+    if (m <= kQgFewRows)
+        return qgemm_few(ctx, w, w_up, ggml_type == CUCA_GGML_Q8_0, k, (kp / 32 / g) * gb, g, x, ldx, m, rows, glu, clamp,
+                         ws, reinterpret_cast<float *>(static_cast<char *>(ws) + xp_bytes), ws_bytes - xp_bytes, out,
+                         out_ld, dtype);
+    const int64_t wide = glu ? 128 : 256; // output columns a workgroup
+    const int64_t n_rt = (rows + wide - 1) / wide;
+    constexpr int tm = 128;
+    const int64_t n_ct = (m + tm - 1) / tm;
     const int64_t tiles = (n_rt + 7) / 8 * 8 * n_ct;
     const int64_t nkc = kp / 128;
     if (tiles > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "qgemm: grid too large");
     // split k for grids smaller than the CU count: up to two workgroups per
-    // CU, at least 4 k-chunks per split, within the workspace given
+    // CU (what the CUs hold at once), at least 4 k-chunks per split, within
+    // the workspace given
     int64_t splits = 1;
     const size_t split_row = (size_t)(glu ? 2 : 1) * (size_t)m * (size_t)rows * 4;
-    if (m <= 2048 && tiles < ctx->cu_count) {
-        splits = std::min<int64_t>(kQgMaxSplits, std::min<int64_t>((2 * ctx->cu_count + tiles - 1) / tiles, nkc / 4));
+    const int64_t work = n_rt * n_ct;
+    if (m <= 2048 && work < ctx->cu_count) {
+        splits = std::min<int64_t>(kQgMaxSplits, std::min<int64_t>(2 * ctx->cu_count / work, nkc / 4));
         splits = std::min<int64_t>(splits, (int64_t)((ws_bytes - xp_bytes) / split_row));
         if (splits < 2) splits = 1;
     }
@@ -2275,38 +2369,24 @@ static cuca_status qgemm_common(cuca_hip_ctx *ctx, const void *w, const void *w_
     a.splits = (int32_t)splits;
     a.clamp = clamp > 0.0f ? clamp : 0.0f;
     a.mp = (int32_t)(n_ct * tm);
+    a.vec = out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (dtype == CUCA_F16 ? 7u : 15u)) == 0;
     const bool f16 = dtype == CUCA_F16, q8 = ggml_type == CUCA_GGML_Q8_0;
     static const Kernel prep_k[2][2] = {{cuca_qgemm_prep_f32_q4_0, cuca_qgemm_prep_f32_q8_0},
                                         {cuca_qgemm_prep_f16_q4_0, cuca_qgemm_prep_f16_q8_0}};
     if ((st = launch(ctx, prep_k[f16][q8], div_up((int64_t)a.mp * nkc * 16, CUCA_BLOCK_THREADS), CUCA_BLOCK_THREADS, 0,
                      a)) != CUCA_OK)
         return st;
-    // [dtype][format][plain, silu, gelu][tokens per tile 32, 64, 128]
-    static const Kernel table_k[2][2][3][3] = {
-        {{{cuca_qgemm_f32_q4_0_t32, cuca_qgemm_f32_q4_0_t64, cuca_qgemm_f32_q4_0_t128},
-          {cuca_qgemm_glu_f32_q4_0_silu_t32, cuca_qgemm_glu_f32_q4_0_silu_t64, cuca_qgemm_glu_f32_q4_0_silu_t128},
-          {cuca_qgemm_glu_f32_q4_0_gelu_t32, cuca_qgemm_glu_f32_q4_0_gelu_t64, cuca_qgemm_glu_f32_q4_0_gelu_t128}},
-         {{cuca_qgemm_f32_q8_0_t32, cuca_qgemm_f32_q8_0_t64, cuca_qgemm_f32_q8_0_t128},
-          {cuca_qgemm_glu_f32_q8_0_silu_t32, cuca_qgemm_glu_f32_q8_0_silu_t64, cuca_qgemm_glu_f32_q8_0_silu_t128},
-          {cuca_qgemm_glu_f32_q8_0_gelu_t32, cuca_qgemm_glu_f32_q8_0_gelu_t64, cuca_qgemm_glu_f32_q8_0_gelu_t128}}},
-        {{{cuca_qgemm_f16_q4_0_t32, cuca_qgemm_f16_q4_0_t64, cuca_qgemm_f16_q4_0_t128},
-          {cuca_qgemm_glu_f16_q4_0_silu_t32, cuca_qgemm_glu_f16_q4_0_silu_t64, cuca_qgemm_glu_f16_q4_0_silu_t128},
-          {cuca_qgemm_glu_f16_q4_0_gelu_t32, cuca_qgemm_glu_f16_q4_0_gelu_t64, cuca_qgemm_glu_f16_q4_0_gelu_t128}},
-         {{cuca_qgemm_f16_q8_0_t32, cuca_qgemm_f16_q8_0_t64, cuca_qgemm_f16_q8_0_t128},
-          {cuca_qgemm_glu_f16_q8_0_silu_t32, cuca_qgemm_glu_f16_q8_0_silu_t64, cuca_qgemm_glu_f16_q8_0_silu_t128},
-          {cuca_qgemm_glu_f16_q8_0_gelu_t32, cuca_qgemm_glu_f16_q8_0_gelu_t64, cuca_qgemm_glu_f16_q8_0_gelu_t128}}}};
-    // [dtype][format][plain, glu][tokens per tile]
-    static const Kernel split_k[2][2][2][3] = {
-        {{{cuca_qgemm_f32_q4_0_t32_split, cuca_qgemm_f32_q4_0_t64_split, cuca_qgemm_f32_q4_0_t128_split},
-          {cuca_qgemm_glu_f32_q4_0_t32_split, cuca_qgemm_glu_f32_q4_0_t64_split, cuca_qgemm_glu_f32_q4_0_t128_split}},
-         {{cuca_qgemm_f32_q8_0_t32_split, cuca_qgemm_f32_q8_0_t64_split, cuca_qgemm_f32_q8_0_t128_split},
-          {cuca_qgemm_glu_f32_q8_0_t32_split, cuca_qgemm_glu_f32_q8_0_t64_split, cuca_qgemm_glu_f32_q8_0_t128_split}}},
-        {{{cuca_qgemm_f16_q4_0_t32_split, cuca_qgemm_f16_q4_0_t64_split, cuca_qgemm_f16_q4_0_t128_split},
-          {cuca_qgemm_glu_f16_q4_0_t32_split, cuca_qgemm_glu_f16_q4_0_t64_split, cuca_qgemm_glu_f16_q4_0_t128_split}},
-         {{cuca_qgemm_f16_q8_0_t32_split, cuca_qgemm_f16_q8_0_t64_split, cuca_qgemm_f16_q8_0_t128_split},
-          {cuca_qgemm_glu_f16_q8_0_t32_split, cuca_qgemm_glu_f16_q8_0_t64_split, cuca_qgemm_glu_f16_q8_0_t128_split}}}};
-    if (splits == 1) return launch(ctx, table_k[f16][q8][glu][ti], (unsigned)tiles, 256, 0, a);
-    if ((st = launch2(ctx, split_k[f16][q8][glu != 0][ti], (unsigned)tiles, (unsigned)splits, 256, 0, a)) != CUCA_OK)
+    // [dtype][format][plain, silu, gelu]
+    static const Kernel table_k[2][2][3] = {
+        {{cuca_qgemm_f32_q4_0, cuca_qgemm_glu_f32_q4_0_silu, cuca_qgemm_glu_f32_q4_0_gelu},
+         {cuca_qgemm_f32_q8_0, cuca_qgemm_glu_f32_q8_0_silu, cuca_qgemm_glu_f32_q8_0_gelu}},
+        {{cuca_qgemm_f16_q4_0, cuca_qgemm_glu_f16_q4_0_silu, cuca_qgemm_glu_f16_q4_0_gelu},
+         {cuca_qgemm_f16_q8_0, cuca_qgemm_glu_f16_q8_0_silu, cuca_qgemm_glu_f16_q8_0_gelu}}};
+    // [format][plain, glu]
+    static const Kernel split_k[2][2] = {{cuca_qgemm_q4_0_split, cuca_qgemm_glu_q4_0_split},
+                                         {cuca_qgemm_q8_0_split, cuca_qgemm_glu_q8_0_split}};
+    if (splits == 1) return launch(ctx, table_k[f16][q8][glu], (unsigned)tiles, 256, 0, a);
+    if ((st = launch2(ctx, split_k[q8][glu != 0], (unsigned)tiles, (unsigned)splits, 256, 0, a)) != CUCA_OK)
         return st;
     static const Kernel red_k[2][3] = {{cuca_qgemm_reduce_f32, cuca_qgemm_reduce_glu_f32_silu, cuca_qgemm_reduce_glu_f32_gelu},
                                        {cuca_qgemm_reduce_f16, cuca_qgemm_reduce_glu_f16_silu, cuca_qgemm_reduce_glu_f16_gelu}};
@@ -2713,7 +2793,8 @@ static cuca_status moe_qgemm_common(cuca_hip_ctx *ctx, const void *w, const void
     const int tm = moe_qgemm_tm(max_pairs, n_experts);
     const int64_t tiles = moe_qgemm_tiles(max_pairs, n_experts, tm);
     const int64_t kp = qgemm_kp(g, k), nkc = kp / 128;
-    const int64_t n_rt = (n + 127) / 128;
+    const int64_t wide = up ? 128 : 256; // output columns a workgroup
+    const int64_t n_rt = (n + wide - 1) / wide;
     const int64_t grid = (n_rt + 7) / 8 * 8 * tiles;
     if (grid > 0x7fffffffll || tiles * tm * nkc * 16 / CUCA_BLOCK_THREADS + 1 > 0x7fffffffll)
         return fail(ctx, CUCA_UNSUPPORTED, "moe qgemm: grid too large");
@@ -2750,6 +2831,7 @@ static cuca_status moe_qgemm_common(cuca_hip_ctx *ctx, const void *w, const void
     a.max_pairs = (int32_t)max_pairs;
     a.tm = tm;
     a.moe_up = up ? 1 : 0;
+    a.vec = out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (up && dtype == CUCA_F16 ? 7u : 15u)) == 0;
     if ((st = launch(ctx, cuca_qgemm_moe_plan, 1, CUCA_BLOCK_THREADS, 0, a)) != CUCA_OK) return st;
     const bool f16 = dtype == CUCA_F16, q8 = ggml_type == CUCA_GGML_Q8_0;
     static const Kernel prep_k[2][2] = {{cuca_qgemm_moe_prep_f32_q4_0, cuca_qgemm_moe_prep_f32_q8_0},

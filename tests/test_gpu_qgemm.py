@@ -128,3 +128,55 @@ def test_qgemm_weight_row_prefix_split_and_errors(ctx):
         ctx.qgemm(wt.packed.ptr, hip.GGML_Q8_0, 300, 4096, dx.ptr, 4096, 40, 100, ws.ptr, small - 256, out.ptr, 100,
                   hip.F32)
     ctx.qgemm(wt.packed.ptr, hip.GGML_Q8_0, 300, 4096, dx.ptr, 4096, 0, 100, ws.ptr, wsb, out.ptr, 100, hip.F32)
+
+
+def run(ctx, wt, qtype, n, k, m, rows, x, ldx, dtype, out_ld, out_off=0, x_off=0):
+    """One call with the activations x_off elements into their buffer and the
+    output out_off into its own; returns the rows and what lies past them."""
+    xb = np.zeros(x_off + m * ldx, NP[dtype])
+    xb[x_off:].reshape(m, ldx)[:, :k] = x
+    ob = np.full(out_off + m * out_ld, 7.0, NP[dtype])
+    dx, out = ctx.array(xb), ctx.array(ob)
+    wsb = hip.qgemm_workspace(QT[qtype], n, k, m)
+    ws = ctx.empty((wsb,), np.uint8)
+    es = np.dtype(NP[dtype]).itemsize
+    ctx.qgemm(wt.packed.ptr, QT[qtype], n, k, dx.ptr + x_off * es, ldx, m, rows, ws.ptr, wsb, out.ptr + out_off * es,
+              out_ld, hip.dtype_code(NP[dtype]))
+    got = out.numpy()
+    return got[out_off:].reshape(m, out_ld)[:, :rows], got[out_off:].reshape(m, out_ld)[:, rows:]
+
+
+@pytest.mark.parametrize("qtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("m", [15, 16, 17, 31, 65, 127, 129, 257])
+@pytest.mark.parametrize("n,rows,k,off", [(1, 1, 32, 0), (65, 63, 480, 1), (129, 129, 544, 3), (260, 257, 3104, 0)])
+def test_qgemm_tile_edges(ctx, qtype, dtype, m, n, rows, k, off):
+    """Both kernels at the edges of their tiles (16, 32, 64 and 128 tokens,
+    128 and 256 weight rows), rows that end inside a packing group (k 32 to
+    3104), a weight-row prefix, activations and outputs `off` elements off
+    their alignment with odd strides, and a canary past every output row."""
+    raw, wt, x = setup(ctx, qtype, n, k, m, dtype, n + k + m)
+    got, past = run(ctx, wt, qtype, n, k, m, rows, x, k + (off or 4), dtype, rows + off, off, off)
+    w = dense(raw, qtype, n, k)[:rows]
+    xf = x.astype(np.float64)
+    want = xf @ w.T
+    tol = bound(xf, w, k) + (2.0 ** -11 * np.abs(want) if dtype == "f16" else 0.0) + 1e-30
+    err = np.abs(got.astype(np.float64) - want)
+    assert np.all(err <= tol), float(np.max(err / tol))
+    assert np.all(past == 7.0)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("m", [8, 200])
+def test_qgemm_over_its_own_activations(ctx, dtype, m):
+    """The output written over the activations it was computed from."""
+    n = k = 512
+    raw, wt, x = setup(ctx, "q4_0", n, k, m, dtype, 11)
+    buf = ctx.array(x)
+    wsb = hip.qgemm_workspace(hip.GGML_Q4_0, n, k, m)
+    ws = ctx.empty((wsb,), np.uint8)
+    ctx.qgemm(wt.packed.ptr, hip.GGML_Q4_0, n, k, buf.ptr, k, m, n, ws.ptr, wsb, buf.ptr, k, hip.dtype_code(NP[dtype]))
+    xf, w = x.astype(np.float64), dense(raw, "q4_0", n, k)
+    want = xf @ w.T
+    tol = bound(xf, w, k) + (2.0 ** -11 * np.abs(want) if dtype == "f16" else 0.0)
+    assert np.all(np.abs(buf.numpy().astype(np.float64) - want) <= tol)
