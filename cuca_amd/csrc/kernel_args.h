@@ -228,6 +228,9 @@ typedef struct {
     void *rn_x_out, *rn_h_out;
     float rn_eps, rn_rs;
     int32_t rn_tpr, rn_per;
+    /* several rows (qms.hip): ntile tiles of tile_rows rows, a tile's rows
+     * cut over js waves; nrb weight blocks of 8 / js waves' rows */
+    int32_t js, tile_rows, gelu, pad3_;
 } QmmArgs;
 
 /* The quantized matmul on the matrix cores (qgemm.hip): out[t][n] =

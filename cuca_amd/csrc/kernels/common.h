@@ -30,6 +30,14 @@ __device__ static inline float pin_f32(float v) {
     return v;
 }
 
+// (w & mask) | magic in one instruction (a gfx9 instruction holds one
+// constant outside its registers, so C code for it compiles to two).
+__device__ static inline uint32_t and_or_b32(uint32_t w, uint32_t mask, uint32_t magic) {
+    uint32_t o;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(o) : "v"(w), "v"(mask), "s"(magic));
+    return o;
+}
+
 template <typename T> struct Chunk;
 
 template <> struct Chunk<float> {

@@ -14,6 +14,7 @@
 #include "pick.hip"
 #include "qmv.hip"
 #include "qmd.hip"
+#include "qms.hip"
 #include "qgemm.hip"
 #include "qgemm_few.hip"
 #include "gemm16.hip"

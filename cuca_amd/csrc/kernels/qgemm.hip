@@ -100,13 +100,6 @@ __device__ static inline void qg_transpose(u32x4 &v) {
     v = u32x4{a[0], a[1], b[0], b[1]};
 }
 
-// (w & mask) | magic in one instruction (a gfx9 instruction holds one
-// constant outside its registers, so C code for it takes two).
-__device__ static inline uint32_t qg_and_or(uint32_t w, uint32_t mask, uint32_t magic) {
-    uint32_t o;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(o) : "v"(w), "v"(mask), "s"(magic));
-    return o;
-}
 __device__ static inline _Float16 qg_scale(qg_u2 s, int i) {
     const uint32_t w = i < 2 ? s.x : s.y;
     return __builtin_bit_cast(_Float16, (uint16_t)((i & 1) ? (w >> 16) : (w & 0xffffu)));
@@ -126,7 +119,7 @@ template <int FMT> __device__ static inline qg_h8 qg_dequant(const QgW<FMT> &w, 
         _Float16 d;
         if (FMT == 0) {
             const uint32_t x = i < 2 ? w.c[0][s] : w.c[0][s] >> 8;
-            v = i & 1 ? qg_and_or(x, 0x00f000f0u, 0x54005400u) : qg_and_or(x, 0x000f000fu, 0x64006400u);
+            v = i & 1 ? and_or_b32(x, 0x00f000f0u, 0x54005400u) : and_or_b32(x, 0x000f000fu, 0x64006400u);
             bias = i & 1 ? 72.0f : 1032.0f;
             d = qg_scale(w.s, i);
         } else { // the biased bytes under 0x64

@@ -61,14 +61,6 @@ template <int FMT> __device__ static inline void qf_load(const uint8_t *grp, int
     for (int i = 0; i < F::G / 8; i++) o.s[i] = *reinterpret_cast<const u32x4 *>(grp + 16 * i);
 }
 
-// (w & mask) | magic in one instruction: written in C the compiler takes two,
-// since a gfx9 instruction holds one constant outside its registers.
-__device__ static inline uint32_t qf_and_or(uint32_t w, uint32_t mask, uint32_t magic) {
-    uint32_t o;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(o) : "v"(w), "v"(mask), "s"(magic));
-    return o;
-}
-
 // The weight operands of the BPD blocks of the exchanged dwords d (element
 // pairs (0,1), (2,3), (16,17), (18,19) past 4u), scales sc: f16(d * q), one
 // rounding.  A nibble is placed under an f16 exponent where it stands: bits
@@ -85,7 +77,7 @@ __device__ static inline void qf_operands(const uint32_t (&d)[4], const _Float16
             float bias;
             if (FMT == 0) {
                 const uint32_t w = i < 2 ? d[p] : d[p] >> 8;
-                v = i & 1 ? qf_and_or(w, 0x00f000f0u, 0x54005400u) : qf_and_or(w, 0x000f000fu, 0x64006400u);
+                v = i & 1 ? and_or_b32(w, 0x00f000f0u, 0x54005400u) : and_or_b32(w, 0x000f000fu, 0x64006400u);
                 bias = i & 1 ? 72.0f : 1032.0f;
             } else {
                 v = __builtin_amdgcn_perm(0x64646464u, d[p], i == 0 ? 0x04020400u : 0x04030401u);

@@ -1532,6 +1532,71 @@ static cuca_status norm_in_launch(cuca_hip_ctx *ctx, const NormIn &rn, int64_t m
                                 rn.h_out, dtype);
 }
 
+// Two rows and more (qms.hip): tiles of up to four rows, evenly filled (5
+// rows: 3 + 2), the tile's rows whole in LDS (160 KB a workgroup at most) and
+// the weight rows addressable by a 32-bit buffer offset.  mode 0: plain / GLU;
+// 3: Q|K|V with RoPE and the K/V store.  Returns false, the call to go to the
+// chunked kernel, where a tile of two rows does not fit.
+constexpr size_t kQmsLds = 160u << 10;
+static size_t qms_lds(int64_t rows, int64_t nbp) { // QMS_LDS_BYTES
+    return (size_t)(rows * (nbp / 4 * 272 + (nbp + 16) * 4) + 4 * 272);
+}
+static bool qms_launch(cuca_hip_ctx *ctx, int mode, int glu, uint32_t ggml_type, int g, cuca_dtype dtype, QmmArgs a,
+                       cuca_status *st) {
+    const int64_t m = a.m, nbp = (int64_t)a.ng * g;
+    if (m < 2 || (int64_t)a.rows * a.row_bytes >= (1ll << 31)) return false;
+    const bool f16 = dtype == CUCA_F16, q8 = ggml_type == CUCA_GGML_Q8_0;
+    int64_t tr = 4;
+    while (tr > 2 && qms_lds(tr, nbp) > kQmsLds) tr--;
+    if (qms_lds(tr, nbp) > kQmsLds) return false;
+    const int64_t ntile = (m + tr - 1) / tr;
+    tr = (m + ntile - 1) / ntile;
+    if (tr < 2) tr = 2;
+    // Two weight rows a lane (gate and up, or a tall matrix) where these give
+    // every compute unit eight waves; otherwise one, the tile's rows cut over
+    // two waves.  At four rows of Q4_0, one / two rows a lane: 6144 x 4096
+    // 15.6 / 20.3 us (768 waves of two), 128256 x 4096 178 / 128 us (16032)
+    const int64_t cus = ctx->cu_count;
+    const bool wide = glu || (mode == 0 && (a.rows + 7) / 8 * ntile >= 8 * cus);
+    // two rows of a matrix of few: the chunked kernel, whose workgroups start
+    // on the weights before the rows are quantised (o at two rows, Q4_0: 7.7
+    // against 8.5 us; down 19.8 against 22.2)
+    if (m == 2 && !wide) return false;
+    a.js = wide ? 1 : tr > 2 ? 2 : 1;
+    if (!wide && tr == 3 && qms_lds(4, nbp) > kQmsLds) { a.js = 1; tr = 2; }
+    a.tile_rows = (int32_t)tr;
+    a.ntile = (int32_t)((m + tr - 1) / tr);
+    a.gelu = glu == 2;
+    // 4 waves a workgroup where 8 leave compute units idle (gate and up of
+    // 3072 x 1024 at four rows: 7.8 -> 6.5 us); 16 where the rows fill a
+    // compute unit's LDS and workgroups of 8 would take turns (4096 x 14336 at
+    // eight rows: 55.5 -> 40.3 us, the chunked kernel 50)
+    int waves = wide ? (glu && (a.rows + 31) / 32 * a.ntile < cus ? 4 : 8) : 4 * a.js;
+    if (!wide && a.js == 2 && qms_lds(4, nbp) > kQmsLds / 2 && (a.rows + 15) / 16 * a.ntile > cus) waves = 16;
+    const int64_t per_wg = waves / a.js * (wide && !glu ? 8 : 4); // weight rows (of each matrix) a workgroup
+    a.nrb = (int32_t)((a.rows + per_wg - 1) / per_wg);
+    const int64_t grid = ((int64_t)a.nrb + 7) / 8 * 8 * a.ntile;
+    if (grid > 0x7fffffffll) return false;
+    static const Kernel wide_k[2][2][3] = {
+        {{cuca_qms_f32_q4_0_w2_j2, cuca_qms_f32_q4_0_w2_j3, cuca_qms_f32_q4_0_w2_j4},
+         {cuca_qms_f32_q8_0_w2_j2, cuca_qms_f32_q8_0_w2_j3, cuca_qms_f32_q8_0_w2_j4}},
+        {{cuca_qms_f16_q4_0_w2_j2, cuca_qms_f16_q4_0_w2_j3, cuca_qms_f16_q4_0_w2_j4},
+         {cuca_qms_f16_q8_0_w2_j2, cuca_qms_f16_q8_0_w2_j3, cuca_qms_f16_q8_0_w2_j4}}};
+    static const Kernel glu_k[2][2][3] = {
+        {{cuca_qms_glu_f32_q4_0_j2, cuca_qms_glu_f32_q4_0_j3, cuca_qms_glu_f32_q4_0_j4},
+         {cuca_qms_glu_f32_q8_0_j2, cuca_qms_glu_f32_q8_0_j3, cuca_qms_glu_f32_q8_0_j4}},
+        {{cuca_qms_glu_f16_q4_0_j2, cuca_qms_glu_f16_q4_0_j3, cuca_qms_glu_f16_q4_0_j4},
+         {cuca_qms_glu_f16_q8_0_j2, cuca_qms_glu_f16_q8_0_j3, cuca_qms_glu_f16_q8_0_j4}}};
+    static const Kernel slim_k[2][2] = {{cuca_qms_f32_q4_0_w1_j2, cuca_qms_f32_q8_0_w1_j2},
+                                        {cuca_qms_f16_q4_0_w1_j2, cuca_qms_f16_q8_0_w1_j2}};
+    static const Kernel rope_k[2][2] = {{cuca_qms_rope_kv_f32_q4_0_j2, cuca_qms_rope_kv_f32_q8_0_j2},
+                                        {cuca_qms_rope_kv_f16_q4_0_j2, cuca_qms_rope_kv_f16_q8_0_j2}};
+    const Kernel k = glu ? glu_k[f16][q8][tr - 2] : wide ? wide_k[f16][q8][tr - 2] : mode == 3 ? rope_k[f16][q8] : slim_k[f16][q8];
+    const int64_t staged = wide ? tr : 2 * a.js;
+    *st = launch(ctx, k, (unsigned)grid, 64u * waves, (unsigned)qms_lds(staged, nbp), a);
+    return true;
+}
+
 // glu: 0 plain, 1 SiLU, 2 GELU-tanh
 static cuca_status qmm_common(cuca_hip_ctx *ctx, const void *w, const void *w_up, uint32_t ggml_type,
                               int64_t n, int64_t k, const void *x, int64_t ldx, int64_t m, int64_t rows,
@@ -1561,13 +1626,14 @@ static cuca_status qmm_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
     if (!al16(x) || ((size_t)ldx * es) % 16 != 0)
         return fail(ctx, CUCA_INVALID_ARG, "qmm: activation rows must start 16-byte aligned");
     const int64_t nb = k / 32, ng = (nb + g - 1) / g;
-    // one or two rows of a tall matrix whose tile fits the LDS: the decode
-    // GEMV stream, each workgroup quantising the rows itself -- except that
-    // one row the one-row kernel takes runs there (measured on MI355X, the
-    // 128256 x 4096 LM head at one row: Q8_0 101-103 -> 88-89 us, Q4_0 59-60
-    // -> 51 us as 8-wave workgroups)
+    // one or two rows of a tall matrix whose tile fits the LDS and that the
+    // one-row and several-row kernels do not take (2 GiB and more): the decode
+    // GEMV stream, each workgroup quantising the rows itself.  Below that the
+    // others are faster (MI355X, the 128256 x 4096 LM head, Q8_0 / Q4_0: one
+    // row 101-103 -> 88-89 us / 59-60 -> 51 us, two rows 131 -> 109 us / 100
+    // -> 88 us)
     const bool qmv = m <= 2 && qmv_wins(ctx, rows) && qmv_fits(m, ng * g, g) &&
-                     !(m == 1 && qmd_fits(m, k, ng, g, rows, ng * gb));
+                     !(m == 1 ? qmd_fits(m, k, ng, g, rows, ng * gb) : rows * ng * gb < (1ll << 31));
     if (qmv) {
         if (rn && (st = norm_in_launch(ctx, *rn, m, k, dtype)) != CUCA_OK) return st;
         return qmv_launch(ctx, 3, w, w_up, ggml_type, n, k, nullptr, 0, nullptr, x, ldx, m, rows, glu, clamp, out,
@@ -1623,6 +1689,7 @@ static cuca_status qmm_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
     const bool fused = rn && qmd && norm_prologue(*rn, m, k, dtype, a);
     if (rn && !fused && (st = norm_in_launch(ctx, *rn, m, k, dtype)) != CUCA_OK) return st;
     if (qmd) return qmd_launch(ctx, 0, glu, ggml_type, k, g, dtype, a, fused);
+    if (qms_launch(ctx, 0, glu, ggml_type, g, dtype, a, &st)) return st;
     return launch(ctx, kk, (unsigned)(nrb8 * ntile), CUCA_BLOCK_THREADS, 0, a);
 }
 
@@ -1706,6 +1773,7 @@ static cuca_status qmm_rope_kv_common(cuca_hip_ctx *ctx, const void *w, uint32_t
     const bool fused = rn && qmd && norm_prologue(*rn, m, k, dtype, a);
     if (rn && !fused && (st = norm_in_launch(ctx, *rn, m, k, dtype)) != CUCA_OK) return st;
     if (qmd) return qmd_launch(ctx, 3, 0, ggml_type, k, g, dtype, a, fused);
+    if (qms_launch(ctx, 3, 0, ggml_type, g, dtype, a, &st)) return st;
     return launch(ctx, table_k[dtype == CUCA_F16][ggml_type == CUCA_GGML_Q8_0][mi], (unsigned)(nrb8 * ntile),
                   CUCA_BLOCK_THREADS, 0, a);
 }

@@ -395,6 +395,30 @@ def test_qkv_rope_store_fused_is_qmm_then_rope_store(ctx, qtype, dtype, nq, nk, 
     qkv_fused_vs_unfused(ctx, rng, qtype, dtype, nq, nk, d, k, m)
 
 
+@pytest.mark.parametrize("qtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("n,k,m", [
+    (1, 32, 3), (31, 96, 4), (33, 1056, 5), (65, 288, 7), (64, 544, 9),     # few rows, tiles of 2 to 4
+    (16385, 96, 2), (16384, 64, 3), (16401, 288, 4), (8200, 64, 5),         # two weight rows a lane
+    (4100, 9216, 4), (2064, 9216, 5),                                       # 16 waves a workgroup
+    (20, 18432, 3), (24, 18432, 5), (9, 36864, 3)])                         # four rows, two rows past the LDS
+def test_several_rows_at_the_edges_of_their_tiles(ctx, qtype, n, k, m):
+    """The oracle's bits at row, block and tile remainders of every split, and
+    a row that holds an infinity or a NaN is what it is alone; the GLU and the
+    fused Q|K|V launch at theirs."""
+    rng = np.random.default_rng(n + k + m)
+    raw, w = weight(ctx, rng, qtype, n, k)
+    x = awkward(rng, m, k, huge=1e4)
+    assert_bits_equal(w.forward(ctx.array(x)).numpy(), want_out(raw, qtype, n, k, x, n, "f32"), f"{n}x{k} m={m}")
+    x[1, 5], x[2 % m, 7] = np.inf, np.nan
+    got = w.forward(ctx.array(x)).numpy()
+    alone = np.concatenate([w.forward(ctx.array(x[j:j + 1])).numpy() for j in range(m)])
+    assert np.array_equal(got, alone, equal_nan=True)
+    if n <= 65 or (n, m) == (8200, 5):
+        test_qmm_glu(ctx, qtype, "f32", hip.ACT_SILU, n, k, m, 0.0)
+    if n <= 33:
+        qkv_fused_vs_unfused(ctx, rng, qtype, "f32", 2, 1, 16, k, m)
+
+
 def test_qkv_rope_store_fused_partial_rotary_bad_slot_and_oracle(ctx):
     rng = np.random.default_rng(77)
     # partial rotary: values past n_dims pass through
