@@ -153,7 +153,7 @@ typedef struct {
     int32_t pad_;
 } RowGatherArgs;
 
-/* Paged attention of many query rows of one sequence (attn_rows.hip): row
+/* Paged attention of many query rows of one sequence (attn_rows.hip, attn_tile.hip): row
  * r of q attends to the positions ranges[r] = [lo, hi) of the sequence's
  * block table.  Values: pool_v, or (pool_v NULL, the latent form) the first
  * v_width columns of the key rows themselves. */

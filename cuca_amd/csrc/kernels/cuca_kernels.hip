@@ -19,3 +19,4 @@
 #include "qgemm_few.hip"
 #include "gemm16.hip"
 #include "attn_rows.hip"
+#include "attn_tile.hip"

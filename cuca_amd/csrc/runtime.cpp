@@ -1237,24 +1237,31 @@ static cuca_status attend_rows_run(cuca_hip_ctx *ctx, const void *q, int64_t q_l
     a.max_blocks = (int32_t)max_blocks;
     a.scale = scale;
     if (mfma) {
-        // [f16][head_dim 64/128/256][group 1/2/4/8]
-        static const Kernel table_k[2][3][4] = {
-            {{cuca_attn_rows_f32_d64_g1, cuca_attn_rows_f32_d64_g2, cuca_attn_rows_f32_d64_g4, cuca_attn_rows_f32_d64_g8},
-             {cuca_attn_rows_f32_d128_g1, cuca_attn_rows_f32_d128_g2, cuca_attn_rows_f32_d128_g4,
-              cuca_attn_rows_f32_d128_g8},
-             {cuca_attn_rows_f32_d256_g1, cuca_attn_rows_f32_d256_g2, cuca_attn_rows_f32_d256_g4,
-              cuca_attn_rows_f32_d256_g8}},
-            {{cuca_attn_rows_f16_d64_g1, cuca_attn_rows_f16_d64_g2, cuca_attn_rows_f16_d64_g4, cuca_attn_rows_f16_d64_g8},
-             {cuca_attn_rows_f16_d128_g1, cuca_attn_rows_f16_d128_g2, cuca_attn_rows_f16_d128_g4,
-              cuca_attn_rows_f16_d128_g8},
-             {cuca_attn_rows_f16_d256_g1, cuca_attn_rows_f16_d256_g2, cuca_attn_rows_f16_d256_g4,
-              cuca_attn_rows_f16_d256_g8}}};
+        if (f16) {
+            // a workgroup: four tiles of 32 (row, query head) pairs of a KV
+            // head, one wave each: up to four heads, then rows
+            static const Kernel tile_k[3][3] = {
+                {cuca_attn_tile_f16_d64_h1, cuca_attn_tile_f16_d64_h2, cuca_attn_tile_f16_d64_h4},
+                {cuca_attn_tile_f16_d128_h1, cuca_attn_tile_f16_d128_h2, cuca_attn_tile_f16_d128_h4},
+                {cuca_attn_tile_f16_d256_h1, cuca_attn_tile_f16_d256_h2, cuca_attn_tile_f16_d256_h4}};
+            const int hw = G < 4 ? G : 4;
+            const int64_t per = 32 * (4 / hw), tiles = (rows + per - 1) / per, wgs = tiles * n_kv * (G / hw);
+            if (wgs > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "too many attention tiles");
+            return launch(ctx, tile_k[di][hw == 4 ? 2 : hw - 1], (unsigned)wgs, 256u, 0u, a);
+        }
+        // [head_dim 64/128/256][group 1/2/4/8]
+        static const Kernel table_k[3][4] = {
+            {cuca_attn_rows_f32_d64_g1, cuca_attn_rows_f32_d64_g2, cuca_attn_rows_f32_d64_g4, cuca_attn_rows_f32_d64_g8},
+            {cuca_attn_rows_f32_d128_g1, cuca_attn_rows_f32_d128_g2, cuca_attn_rows_f32_d128_g4,
+             cuca_attn_rows_f32_d128_g8},
+            {cuca_attn_rows_f32_d256_g1, cuca_attn_rows_f32_d256_g2, cuca_attn_rows_f32_d256_g4,
+             cuca_attn_rows_f32_d256_g8}};
         // a workgroup: RT tiles of 16 rows x the G query heads, one wave each
         // (the kernels' launch shape: RT = 4 at groups 1 and 2, 8 / G beyond)
         const int rt = G <= 2 ? 4 : 8 / G;
         const int64_t tiles = (rows + 16 * rt - 1) / (16 * rt);
         if (tiles * n_kv > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "too many attention tiles");
-        return launch(ctx, table_k[f16][di][gi], (unsigned)(tiles * n_kv), (unsigned)(64 * G * rt), 0u, a);
+        return launch(ctx, table_k[di][gi], (unsigned)(tiles * n_kv), (unsigned)(64 * G * rt), 0u, a);
     }
     const int64_t jobs = rows * n_head;
     if ((jobs + 3) / 4 > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "too many attention rows");

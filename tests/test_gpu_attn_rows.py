@@ -189,6 +189,32 @@ def test_a_missing_block_past_the_first_table_window_is_reported(ctx, dtype):
     assert_close(got[16:], want, floor=floor_of(table, ranges[16:], pv, nq), what="rows after the block")
 
 
+@pytest.mark.parametrize("nq,nk,d,t,start,scale", [
+    (2, 2, 64, 1, 0, 0.1), (4, 2, 64, 65, 62, -0.1), (8, 1, 64, 33, 1023, 0.1),      # a key; tile and head-group
+    (4, 1, 128, 32, 32, 0.1), (8, 1, 128, 31, 992, 0.0), (3, 3, 128, 129, 0, 0.1),   # edges; the end of the first
+    (2, 1, 128, 63, 1090, -0.1), (1, 1, 256, 40, 1000, 0.1), (8, 1, 256, 34, 30, 0.1)])  # 64 table entries
+def test_f16_tiles_at_their_edges(ctx, nq, nk, d, t, start, scale):
+    """Row tiles of 32 and key tiles of 64 with remainders, causal and with a
+    window, negative and zero scales, values outside a row's range that are
+    not finite (the row does not see them), a row alone and in its chunk."""
+    rng = np.random.default_rng(nq + d + t + start)
+    n_blocks = (t + start + 15) // 16 + 3
+    pk, pv = (rng.standard_normal((n_blocks, nk, 16, d)).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((t, nq, d)).astype(np.float16)
+    for window in (None, 70):
+        table, ranges = chunk(rng, t, start, n_blocks, n_blocks, window)
+        all_rows = check(ctx, q, pk, pv, table, ranges, nq, scale)
+        one = run_rows(ctx, q[t // 2:t // 2 + 1], pk, pv, table, ranges[t // 2:t // 2 + 1], nq, scale)
+        assert_bits_equal(one[0], all_rows[t // 2], "a row alone")
+        # the last position's value, in the last row's range alone
+        last, bad = t + start - 1, pv.copy()
+        bad[table[last // 16], :, last % 16, ::2] = np.inf
+        bad[table[last // 16], :, last % 16, 1::2] = np.nan
+        got = run_rows(ctx, q, pk, bad, table, ranges, nq, scale)
+        assert_close(got[:-1], all_rows[:-1], floor=floor_of(table, ranges[:-1], pv, nq), what="rows before it")
+        assert not np.isfinite(got[-1].astype(np.float32)).any()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
 @pytest.mark.parametrize("nh,d,vw,t", [(16, 576, 512, 21), (4, 80, 64, 33)])
 def test_latent_rows(ctx, dtype, nh, d, vw, t):
