@@ -327,17 +327,17 @@ typedef struct {
     int32_t m, nb;
 } Q8ActsArgs;
 
-/* The decode GEMV (qmv.hip): tiles of MT <= 4 activation rows held in LDS
- * for the whole row length, either quantised already (quants / scales) or
- * quantised by the workgroup from x; tasks of 4 weight rows per wave.
- * Epilogue as QmmArgs (GLU, cap).  MoE (modes 1 / 2): workgroup (tile,
- * split) takes tile `tile` of the expert order and row tasks
- * [split * tps, (split + 1) * tps) of the expert's matrix. */
+/* The decode GEMV (qmv.hip): one or two activation rows held in LDS for the
+ * whole row length, either quantised already (quants / scales) or quantised
+ * by the workgroup from x; tasks of 4 weight rows per wave.  Epilogue as
+ * QmmArgs (GLU, cap).  The routed experts at decode (qms_moe.hip): workgroup
+ * (tile, split) takes tile `tile` (of up to m pairs) of the expert order and
+ * row tasks [split * tps, (split + 1) * tps) of the expert's matrix. */
 typedef struct {
     const uint8_t *w, *w_up;    /* packed weights (gate/up for GLU)          */
     const int8_t *quants;       /* mode 0: [m][q_ld]                         */
     const float *scales;        /* mode 0: [m][nb]                           */
-    const void *x;              /* modes 1-3: activation rows [.][ldx]       */
+    const void *x;              /* mode 3, MoE: activation rows [.][ldx]       */
     void *out;                  /* [m or pairs][out_ld]                      */
     const int32_t *offsets;     /* MoE: [n_experts + 1]                      */
     const int32_t *pair_token;  /* MoE up: [max_pairs]                       */
@@ -349,6 +349,7 @@ typedef struct {
     float clamp;
     int32_t cap_flags;
     float mul1, mul2, softcap_inv, softcap;
+    int32_t gelu;               /* MoE up: GELU-tanh, else SiLU              */
 } QmvArgs;
 
 /* Greedy argmax and top-k over logits rows (sampler.rs greedy and

@@ -15,6 +15,7 @@
 #include "qmv.hip"
 #include "qmd.hip"
 #include "qms.hip"
+#include "qms_moe.hip"
 #include "qgemm.hip"
 #include "qgemm_few.hip"
 #include "gemm16.hip"

@@ -69,7 +69,11 @@ template <int MJ> __device__ static inline void qms_dots(uint32_t w, const uint3
 }
 template <int MJ>
 __device__ static inline void qms_dots2(uint32_t w, uint32_t u, const uint32_t (&x)[MJ], float (&o)[MJ], float (&p)[MJ]) {
-    if constexpr (MJ == 2)
+    if constexpr (MJ == 1)
+        asm("v_dot2_f32_f16 %0, %2, %4, 0\n\tv_dot2_f32_f16 %1, %3, %4, 0\n\ts_nop 2"
+            : "=&v"(o[0]), "=&v"(p[0])
+            : "v"(w), "v"(u), "v"(x[0]));
+    else if constexpr (MJ == 2)
         asm("v_dot2_f32_f16 %0, %4, %6, 0\n\tv_dot2_f32_f16 %1, %4, %7, 0\n\t"
             "v_dot2_f32_f16 %2, %5, %6, 0\n\tv_dot2_f32_f16 %3, %5, %7, 0\n\ts_nop 2"
             : "=&v"(o[0]), "=&v"(o[1]), "=&v"(p[0]), "=&v"(p[1])

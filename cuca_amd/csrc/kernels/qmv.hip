@@ -1,7 +1,6 @@
 // qmv.hip -- the decode GEMV of the CPU engine's quantized matmul (qmm.rs)
-// on gfx950: the same bits as qmm.hip, for one to four activation rows,
-// shaped for the latency of a decode step, and the routed experts (MoE) at
-// decode on the same kernel.
+// on gfx950: the same bits as qmm.hip, for one or two activation rows,
+// shaped for the latency of a decode step.
 //
 // A workgroup holds its activation rows for the whole row length in LDS,
 // expanded once to what the integer dot reads: the f16 pair and C of
@@ -9,21 +8,14 @@
 //   mode 0: quantised already (cuca_q8_acts_*: Acts::new, qmm.rs:1217-1343,
 //           one thread per 32 values), shared by every workgroup;
 //   mode 3: as f32 / f16 values, quantised by the workgroup (Acts::new,
-//           the same bits), so a call is one launch;
-//   mode 1 (MoE up) / 2 (MoE down): the rows of one tile of an expert's
-//           pairs (up: the pairs' token rows of x; down: the pairs' hidden
-//           rows), quantised by the workgroup.
+//           the same bits), so a call is one launch.
 // Its four waves then run independently.  A wave's task is four weight rows
 // x sixteen lanes, each thread one chain over all blocks; a wave takes a
 // sequence of tasks and streams their groups of G blocks back to back
 // through a ring of QMV_D groups in flight, so the next task's weights load
 // while the current one finishes.  Per group a wave stages dw * dx of its
 // four rows in its own LDS area (no workgroup barrier).
-// Modes 0 / 3: workgroups are persistent, a wave's tasks are strided over
-// the grid.  Modes 1 / 2: workgroup (tile, split) takes tile `tile` of the
-// expert order (moe_tile_lookup) and a contiguous range of the expert's row
-// tasks; the outputs are those of the one-pass MoE kernels (hidden rows in
-// pair order; f32 rows y * routing weight for moe_sum).
+// Workgroups are persistent, a wave's tasks are strided over the grid.
 #include "common.h"
 
 #define QMV_WAVES 4
@@ -118,14 +110,12 @@ __device__ static inline void qmv_load(const uint8_t *w, int g, int l, u32x4 &ch
 }
 __device__ static inline float qmv_scale(uint32_t pair, int l) { return qmv_h2f(pair >> (16 * (l & 1))); }
 
-// MODE 0: quantised rows (a.quants / a.scales), dense; 3: dense rows of
-// a.x; 1: MoE up; 2: MoE down.  TX: the activation type (modes 1-3); TO:
-// the output type.
+// MODE 0: quantised rows (a.quants / a.scales); 3: rows of a.x.  TX: the
+// activation type (mode 3); TO: the output type.
 template <int FMT, int MT, bool GLU, int ACT, typename TX, typename TO, int MODE>
 __device__ static inline void qmv_body(const QmvArgs &a) {
     using F = QFmt<FMT>;
     constexpr int G = F::G;
-    constexpr bool MOE = MODE == 1 || MODE == 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char qmv_lds[];
     const int xstr = a.nbp + 2;
     qmm_u2 *xe = reinterpret_cast<qmm_u2 *>(qmv_lds);
@@ -136,27 +126,9 @@ __device__ static inline void qmv_body(const QmvArgs &a) {
     const int tid = threadIdx.x, lt = tid % CUCA_WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / CUCA_WAVE);
 
-    // the tile's rows and weights; the wave's tasks first, first + step, ... < tend
+    // the wave's tasks first, first + step, ... < tend
     const uint8_t *wm = a.w, *um = a.w_up;
-    int p0 = 0, np = a.m, first, step, tend;
-    if constexpr (MOE) {
-        const int tile = blockIdx.x / a.splits, split = blockIdx.x - tile * a.splits;
-        int e, q0, q1;
-        if (!moe_tile_lookup<MT>(a.offsets, a.n_experts, a.max_pairs, tile, &e, &q0, &q1)) return;
-        e = __builtin_amdgcn_readfirstlane(e);
-        p0 = __builtin_amdgcn_readfirstlane(q0);
-        np = __builtin_amdgcn_readfirstlane(q1) - p0;
-        wm = a.w + (int64_t)e * a.w_estride;
-        um = GLU ? a.w_up + (int64_t)e * a.w_estride : nullptr;
-        const int t0 = split * a.tps;
-        first = t0 + wave;
-        step = QMV_WAVES;
-        tend = min(a.ntask, t0 + a.tps);
-    } else {
-        first = blockIdx.x * QMV_WAVES + wave;
-        step = gridDim.x * QMV_WAVES;
-        tend = a.ntask;
-    }
+    const int first = blockIdx.x * QMV_WAVES + wave, step = gridDim.x * QMV_WAVES, tend = a.ntask;
 
     // expand the tile's rows: (f16 pair, C) per (row, lane, block), scales
     if constexpr (MODE == 0) {
@@ -179,20 +151,10 @@ __device__ static inline void qmv_body(const QmvArgs &a) {
     } else {
         for (int e = tid; e < MT * a.nbp; e += QMV_WAVES * CUCA_WAVE) {
             const int j = e / a.nbp, b = e - j * a.nbp;
-            int64_t xr = -1;
-            if (j < np && b < a.nb) {
-                if (MODE == 1) {
-                    const int t = a.pair_token[p0 + j];
-                    if (t >= 0 && t < a.n_tokens) xr = (int64_t)t * a.ldx;
-                    else if (b == 0) record_bad(a.status + CUCA_STATUS_MOE_PAIR, (uint32_t)(p0 + j), (uint32_t)t);
-                } else {
-                    xr = (int64_t)(p0 + j) * a.ldx;
-                }
-            }
             float v[32];
             float d = 0.0f;
-            if (xr >= 0) {
-                qmv_load32<TX>(reinterpret_cast<const TX *>(a.x) + xr + (int64_t)b * 32, v);
+            if (j < a.m && b < a.nb) {
+                qmv_load32<TX>(reinterpret_cast<const TX *>(a.x) + (int64_t)j * a.ldx + (int64_t)b * 32, v);
                 d = qmv_quant_block(v);
             } else {
 #pragma unroll
@@ -203,18 +165,6 @@ __device__ static inline void qmv_body(const QmvArgs &a) {
         }
     }
     __syncthreads();
-
-    // which of the tile's rows have outputs (MoE up: a valid token)
-    uint32_t jmask = 0;
-#pragma unroll
-    for (int j = 0; j < MT; j++) {
-        bool v = j < np;
-        if (MODE == 1 && v) {
-            const int t = a.pair_token[p0 + j];
-            v = t >= 0 && t < a.n_tokens;
-        }
-        jmask |= v ? 1u << j : 0u;
-    }
 
     const int nt = first < tend ? (tend - first + step - 1) / step : 0;
     if (nt == 0) return;
@@ -337,7 +287,7 @@ __device__ static inline void qmv_body(const QmvArgs &a) {
         for (int e = lt; e < cn * MT * 4; e += CUCA_WAVE) {
             const int ti = e / (MT * 4), j = (e / 4) % MT, rr = e % 4;
             const int row = (first + (c0 + ti) * step) * 4 + rr;
-            if (row >= a.rows || !((jmask >> j) & 1u)) continue;
+            if (row >= a.rows || j >= a.m) continue;
             float o = res[((ti * MT + j) * 2) * 4 + rr];
             if (GLU) {
                 float gg = o, u = res[((ti * MT + j) * 2 + 1) * 4 + rr];
@@ -346,15 +296,12 @@ __device__ static inline void qmv_body(const QmvArgs &a) {
                     u = fminf(fmaxf(u, -a.clamp), a.clamp);
                 }
                 o = (ACT == 0 ? act_silu(gg) : act_gelu_tanh(gg)) * u;
-            } else if (!MOE && a.cap_flags) { // cap_logits (cpu.rs:2603-2617)
+            } else if (a.cap_flags) { // cap_logits (cpu.rs:2603-2617)
                 if (a.cap_flags & 1) o = o * a.mul1 + 0.0f;
                 if (a.cap_flags & 2) o = o * a.mul2 + 0.0f;
                 if (a.cap_flags & 4) o = tanhf(o * a.softcap_inv + 0.0f) * a.softcap + 0.0f;
             }
-            if (MODE == 2) // CpuExpert::add_picks: y * weight (cpu.rs:400-417)
-                reinterpret_cast<float *>(a.out)[(int64_t)(p0 + j) * a.out_ld + row] = o * a.pair_weight[p0 + j];
-            else
-                reinterpret_cast<TO *>(a.out)[(int64_t)(p0 + j) * a.out_ld + row] = to_stored<TO>(o);
+            reinterpret_cast<TO *>(a.out)[(int64_t)j * a.out_ld + row] = to_stored<TO>(o);
         }
         __builtin_amdgcn_wave_barrier();
     }
@@ -380,20 +327,3 @@ CUCA_QMV_SET(q4_0, 0, 1, f16, _Float16)
 CUCA_QMV_SET(q4_0, 0, 2, f16, _Float16)
 CUCA_QMV_SET(q8_0, 1, 1, f16, _Float16)
 CUCA_QMV_SET(q8_0, 1, 2, f16, _Float16)
-// MoE at decode: tiles of 1, 2 or 4 pairs
-#define CUCA_QMV_MOE_SET(FN, FMT, MT, TN, T)                                               \
-    CUCA_QMV(cuca_qmv_moe_up_##FN##_silu_m##MT##_##TN, FMT, MT, true, 0, T, T, 1)          \
-    CUCA_QMV(cuca_qmv_moe_up_##FN##_gelu_m##MT##_##TN, FMT, MT, true, 1, T, T, 1)          \
-    CUCA_QMV(cuca_qmv_moe_down_##FN##_m##MT##_##TN, FMT, MT, false, 0, T, float, 2)
-CUCA_QMV_MOE_SET(q4_0, 0, 1, f32, float)
-CUCA_QMV_MOE_SET(q4_0, 0, 2, f32, float)
-CUCA_QMV_MOE_SET(q4_0, 0, 4, f32, float)
-CUCA_QMV_MOE_SET(q8_0, 1, 1, f32, float)
-CUCA_QMV_MOE_SET(q8_0, 1, 2, f32, float)
-CUCA_QMV_MOE_SET(q8_0, 1, 4, f32, float)
-CUCA_QMV_MOE_SET(q4_0, 0, 1, f16, _Float16)
-CUCA_QMV_MOE_SET(q4_0, 0, 2, f16, _Float16)
-CUCA_QMV_MOE_SET(q4_0, 0, 4, f16, _Float16)
-CUCA_QMV_MOE_SET(q8_0, 1, 1, f16, _Float16)
-CUCA_QMV_MOE_SET(q8_0, 1, 2, f16, _Float16)
-CUCA_QMV_MOE_SET(q8_0, 1, 4, f16, _Float16)

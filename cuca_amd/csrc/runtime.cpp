@@ -2646,36 +2646,33 @@ static cuca_status moe_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
     const double mean = (double)max_pairs / (double)n_experts;
     const int mt = mean <= 1.5 ? 1 : mean <= 3.0 ? 2 : 4;
     const int mi = mt == 1 ? 0 : mt == 2 ? 1 : 2;
-    // an upper bound of the tiles, sum over experts of ceil(n_e / mt): at
+    // an upper bound of the tiles, sum over experts of ceil(n_e / t): at
     // most min(n_experts, pairs) experts hold pairs, each adding at most
-    // (mt - 1) / mt of a tile to pairs / mt
-    const int64_t ntile = (max_pairs + (mt - 1) * std::min<int64_t>(n_experts, max_pairs)) / mt;
-    // the decode GEMV, a workgroup per (tile, split of the expert's rows),
-    // when the tile's rows fit its LDS, from two tokens' pairs up (16 pairs
-    // over 128 experts; measured at Qwen3-30B-A3B's shapes: 34 vs 36 us at
-    // two tokens, 159 vs 448 us at 32); a single token's pairs keep the
-    // one-pass kernel (25 vs 30 us)
-    if (16 * max_pairs > n_experts && qmv_lds(mt, ng * g, g) <= (64u << 10)) {
-        const int64_t ntask = (n + 3) / 4;
-        int64_t splits = std::max<int64_t>(1, ((int64_t)ctx->cu_count * 4 + ntile - 1) / ntile);
+    // (t - 1) / t of a tile to pairs / t
+    auto tiles = [&](int64_t t) { return (max_pairs + (t - 1) * std::min<int64_t>(n_experts, max_pairs)) / t; };
+    // qms_moe.hip, a workgroup per (tile, split of the expert's rows), from
+    // two tokens' pairs up (16 pairs over 128 experts); a single token's
+    // pairs keep the one-pass kernel.  Tiles of four pairs where two such
+    // workgroups fit a compute unit's LDS, of fewer (for longer rows) where
+    // the experts hold no more on average; otherwise the one-pass kernel
+    auto lds = [&](int64_t t) { return qms_lds(t, ng * g) + (size_t)t * 4 * 16 * 8 * 4; }; // QMS_MOE_LDS_BYTES
+    const int64_t tr = lds(4) <= (80u << 10) ? 4 : mt <= 2 && lds(2) <= (80u << 10) ? 2
+                                             : mt == 1 && lds(1) <= (80u << 10) ? 1 : 0;
+    if (16 * max_pairs > n_experts && tr && packed < (1ll << 31)) {
+        const int64_t nt = tiles(tr), ntask = up ? (n + 3) / 4 : (n + 7) / 8;
+        // eight workgroups a compute unit by the tile bound (about half of it
+        // is there at 32 tokens; at 2 / 4 / 8 / 16: 127, 127, 115, 125 us), in
+        // eights: blockIdx % 8 is the XCD, so a split of all an expert's
+        // tiles reads its rows from one L2
+        int64_t splits = (((int64_t)ctx->cu_count * 8 + nt - 1) / nt + 7) / 8 * 8;
         splits = std::min<int64_t>(splits, (ntask + 3) / 4);
         const int64_t tps = ((ntask + splits - 1) / splits + 3) / 4 * 4;
-        splits = (ntask + tps - 1) / tps;
-        if (ntile * splits > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "moe: grid too large");
-        // [dtype][format][up silu, up gelu, down][tile rows 1, 2, 4]
-        static const Kernel table_v[2][2][3][3] = {
-            {{{cuca_qmv_moe_up_q4_0_silu_m1_f32, cuca_qmv_moe_up_q4_0_silu_m2_f32, cuca_qmv_moe_up_q4_0_silu_m4_f32},
-              {cuca_qmv_moe_up_q4_0_gelu_m1_f32, cuca_qmv_moe_up_q4_0_gelu_m2_f32, cuca_qmv_moe_up_q4_0_gelu_m4_f32},
-              {cuca_qmv_moe_down_q4_0_m1_f32, cuca_qmv_moe_down_q4_0_m2_f32, cuca_qmv_moe_down_q4_0_m4_f32}},
-             {{cuca_qmv_moe_up_q8_0_silu_m1_f32, cuca_qmv_moe_up_q8_0_silu_m2_f32, cuca_qmv_moe_up_q8_0_silu_m4_f32},
-              {cuca_qmv_moe_up_q8_0_gelu_m1_f32, cuca_qmv_moe_up_q8_0_gelu_m2_f32, cuca_qmv_moe_up_q8_0_gelu_m4_f32},
-              {cuca_qmv_moe_down_q8_0_m1_f32, cuca_qmv_moe_down_q8_0_m2_f32, cuca_qmv_moe_down_q8_0_m4_f32}}},
-            {{{cuca_qmv_moe_up_q4_0_silu_m1_f16, cuca_qmv_moe_up_q4_0_silu_m2_f16, cuca_qmv_moe_up_q4_0_silu_m4_f16},
-              {cuca_qmv_moe_up_q4_0_gelu_m1_f16, cuca_qmv_moe_up_q4_0_gelu_m2_f16, cuca_qmv_moe_up_q4_0_gelu_m4_f16},
-              {cuca_qmv_moe_down_q4_0_m1_f16, cuca_qmv_moe_down_q4_0_m2_f16, cuca_qmv_moe_down_q4_0_m4_f16}},
-             {{cuca_qmv_moe_up_q8_0_silu_m1_f16, cuca_qmv_moe_up_q8_0_silu_m2_f16, cuca_qmv_moe_up_q8_0_silu_m4_f16},
-              {cuca_qmv_moe_up_q8_0_gelu_m1_f16, cuca_qmv_moe_up_q8_0_gelu_m2_f16, cuca_qmv_moe_up_q8_0_gelu_m4_f16},
-              {cuca_qmv_moe_down_q8_0_m1_f16, cuca_qmv_moe_down_q8_0_m2_f16, cuca_qmv_moe_down_q8_0_m4_f16}}}};
+        if (tps * splits > 0x7fffffffll || nt * splits > 0x7fffffffll)
+            return fail(ctx, CUCA_UNSUPPORTED, "moe: grid too large");
+        // [dtype][format][down, up]
+        static const Kernel table_s[2][2][2] = {
+            {{cuca_qms_moe_down_f32_q4_0, cuca_qms_moe_up_f32_q4_0}, {cuca_qms_moe_down_f32_q8_0, cuca_qms_moe_up_f32_q8_0}},
+            {{cuca_qms_moe_down_f16_q4_0, cuca_qms_moe_up_f16_q4_0}, {cuca_qms_moe_down_f16_q8_0, cuca_qms_moe_up_f16_q8_0}}};
         QmvArgs v{};
         v.w = static_cast<const uint8_t *>(w);
         v.w_up = static_cast<const uint8_t *>(w_up);
@@ -2690,7 +2687,7 @@ static cuca_status moe_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
         v.w_estride = estride;
         v.row_bytes = ng * gb;
         v.rows = (int32_t)n;
-        v.m = mt;
+        v.m = (int32_t)tr;
         v.nb = (int32_t)nb;
         v.ng = (int32_t)ng;
         v.nbp = (int32_t)(ng * g);
@@ -2701,10 +2698,12 @@ static cuca_status moe_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
         v.splits = (int32_t)splits;
         v.tps = (int32_t)tps;
         v.clamp = clamp > 0.0f ? clamp : 0.0f;
+        v.gelu = up == 2;
         if (up) ctx->last_moe_tokens = n_tokens;
-        return launch(ctx, table_v[dtype == CUCA_F16][ggml_type == CUCA_GGML_Q8_0][up ? up - 1 : 2][mi],
-                      (unsigned)(ntile * splits), CUCA_BLOCK_THREADS, (unsigned)qmv_lds(mt, ng * g, g), v);
+        return launch(ctx, table_s[dtype == CUCA_F16][ggml_type == CUCA_GGML_Q8_0][up ? 1 : 0],
+                      (unsigned)(nt * splits), CUCA_BLOCK_THREADS, (unsigned)lds(tr), v);
     }
+    const int64_t ntile = tiles(mt);
     const int64_t nrb = (n + 15) / 16, nrb8 = (nrb + 7) / 8 * 8;
     if (nrb8 * ntile > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "moe: grid too large");
     // [dtype][format][up silu, up gelu, down][tile rows 1, 2, 4]

@@ -16,7 +16,8 @@ Bars:
   f16 activations round the hidden rows to f16 (the reference is f32
   throughout), checked to 1e-2 as a sanity bound only.
 Covers Q4_0 / Q8_0, f32 / f16, SiLU / GELU-tanh, both kernels (the decode
-GEMV, and the one-pass kernel for rows too long for its LDS: hidden 8192),
+kernel, and the one-pass kernel for rows too long for its LDS: hidden 8192),
+every fill of the decode kernel's tiles,
 experts with no pairs,
 Zipf(1.1) routing over 128 experts at the Qwen3-30B-A3B shapes (decode
 batch 64, top 8), and a pair token outside the rows (reported, skipped).
@@ -130,6 +131,50 @@ def test_moe_layer(ctx, qtype, dtype, act, t, n_experts, n_used, n_embd, ff):
     assert np.all(np.abs(got.astype(np.float64) - want) <= (1e-4 if dtype == "f32" else 1e-2) * scale)
 
 
+# pairs per expert, weight rows, row length: tiles of four (full and of one to
+# three pairs), rows that are no multiple of a task's, one group and partial
+# groups of blocks, several tasks' chunks a wave; tiles of two and of one where
+# the rows are long and the experts hold few pairs
+@pytest.mark.parametrize("qtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("counts,rows,k", [([1, 0, 2, 3, 4, 5, 7, 9], 37, 544), ([3, 4], 4, 32),
+                                           ([1, 2, 3, 4] * 64, 1029, 96), ([3, 0, 1, 2, 0, 1, 4, 0], 29, 12288),
+                                           ([3, 0, 1, 2, 0, 1, 4, 0], 13, 20480)])
+def test_decode_kernel_tiles(ctx, qtype, dtype, counts, rows, k):
+    rng = np.random.default_rng(rows + k)
+    npd = np.float16 if dtype == "f16" else np.float32
+    E, pairs, few = len(counts), sum(counts), min(len(counts), 8)
+    raws = [[W.quant_table(rng, rows, k, qtype, (0.002, 0.01)) for _ in range(3)] for _ in range(few)]
+    one = (hip.qweight_bytes(QT[qtype], rows, k) + 15) // 16 * 16
+    pools = [ctx.empty((E * one,), np.uint8) for _ in range(3)]
+    for e in range(E):
+        for pool, raw in zip(pools, raws[e % few]):
+            d = ctx.array(raw)
+            ctx.qweight_pack(d.ptr, QT[qtype], rows, k, pool.ptr + e * one)
+            ctx.sync()
+    x = (rng.standard_normal((pairs, k)) * min(1.0, np.sqrt(256.0 / k))).astype(npd)
+    tok = rng.permutation(pairs).astype(np.int32)
+    wt = rng.uniform(0.05, 1.0, pairs).astype(np.float32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    dx, d_off, d_tok, d_wt = (ctx.array(v) for v in (x, offsets, tok, wt))
+    hidden, scr = ctx.empty((pairs, rows), npd), ctx.empty((pairs, rows), np.float32)
+    ctx.moe_up(pools[0].ptr, pools[1].ptr, one, QT[qtype], rows, k, E, dx.ptr, k, pairs, d_off.ptr, d_tok.ptr, pairs,
+               hip.ACT_SILU, 0.0, hidden.ptr, rows, hip.dtype_code(npd))
+    ctx.moe_down(pools[2].ptr, one, QT[qtype], rows, k, E, dx.ptr, k, d_off.ptr, d_wt.ptr, pairs, scr.ptr, rows,
+                 hip.dtype_code(npd))
+    got_h, got_s = hidden.numpy(), scr.numpy()
+    for e in range(E):
+        lo, hi = offsets[e], offsets[e + 1]
+        if lo == hi:
+            continue
+        gate, up, down = raws[e % few]
+        xr = x[tok[lo:hi]].astype(np.float32)
+        wh = O.glu(O.qmm(gate, QT[qtype], rows, k, xr), O.qmm(up, QT[qtype], rows, k, xr), hip.ACT_SILU)
+        assert_close(got_h[lo:hi], wh.astype(npd), what=f"moe_up expert {e}")
+        y = O.qmm(down, QT[qtype], rows, k, x[lo:hi].astype(np.float32))
+        assert_bits_equal(got_s[lo:hi], (y * wt[lo:hi, None]).astype(np.float32), f"moe_down expert {e}")
+
+
 def test_moe_sum_adds_in_the_given_order(ctx):
     """2^30, 1, -2^30 summed in order from 0 is 0 (2^30 + 1 rounds to 2^30);
     the order 2^30, -2^30, 1 gives 1, and -2^30, (none), 1 gives -2^30."""
@@ -163,7 +208,7 @@ def test_qwen3_30b_a3b_shapes_zipf_routing(ctx):
 
 @pytest.mark.parametrize("n_experts", [4, 128])
 def test_a_pair_token_outside_the_rows_is_reported(ctx, n_experts):
-    """On both kernels: the decode GEMV (4 pairs over 4 experts) and the
+    """On both kernels: the decode kernel (4 pairs over 4 experts) and the
     one-pass kernel (4 pairs over 128 experts)."""
     rng = np.random.default_rng(9)
     experts, eb = bank(ctx, rng, "q8_0", n_experts, 64, 32)
