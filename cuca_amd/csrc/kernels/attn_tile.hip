@@ -156,8 +156,6 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
             offv[i] = key * RB + ((slot ^ vx) << 4);
         }
         const int wblk = wave * (KT / 4) / 16; // the wave's block of a tile
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
         auto copy = [&](auto IV, int t) { // tile t of K (0) or V (1) into its buffer
             constexpr int V = IV.value;
             uint32_t blk = (uint32_t)__builtin_amdgcn_readlane((int)tabv, (t - tw) * NB + wblk);
@@ -168,11 +166,9 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
 #pragma unroll
             for (int i = 0; i < NC; i++) {
                 const uint32_t dst = (uint32_t)(uintptr_t)&kv[t & 1][V][(wave * (KT / 4) + RPC * i) * RB];
-                asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off[i]), "s"(src), "s"(dst)
-                             : "memory", "m0");
+                lds_copy16(off[i], src, dst);
             }
         };
-#pragma clang diagnostic pop
         // operand addresses within a buffer
         const int kx = (D == 64 ? (c >> 1) & 7 : c & 15);
         uint32_t ka[NJ], va[ND];

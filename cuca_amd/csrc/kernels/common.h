@@ -38,6 +38,27 @@ __device__ static inline uint32_t and_or_b32(uint32_t w, uint32_t mask, uint32_t
     return o;
 }
 
+// A wave's copy of 16 bytes a lane straight into LDS: lane L's bytes at src +
+// off(L) go to LDS dst + 16 L (src and dst uniform).  From inline assembly with
+// the waits written out by the caller: the compiler cannot tell several LDS
+// buffers apart behind such a copy and would wait for every copy in flight
+// before any LDS read.  M0, the copy's LDS base, is set by the same statement
+// (clang warns that the clobber names a reserved register), and the hardware
+// wants one wait state between a scalar write of M0 and the copy that reads
+// it: the compiler puts it after its own writes but not inside an asm string,
+// so it is written here.  SC0: the cache policy bit of that name.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+template <bool SC0 = false> __device__ static inline void lds_copy16(uint32_t off, uint64_t src, uint32_t dst) {
+    if constexpr (SC0)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 sc0" ::"v"(off), "s"(src), "s"(dst)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(src), "s"(dst)
+                     : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 template <typename T> struct Chunk;
 
 template <> struct Chunk<float> {

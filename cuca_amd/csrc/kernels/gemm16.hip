@@ -130,26 +130,18 @@ __device__ static inline void gemm16_body(const Gemm16Args &a) {
         if (lr >= lim) lr = 0;
         off[i] = 2u * ((uint32_t)lr * ld + 8u * (uint32_t)pu);
     }
-    // The copies are issued from inline assembly, with the explicit waits
-    // below: the compiler cannot tell the four buffers apart behind an LDS
-    // DMA and would otherwise wait for every copy in flight before any LDS
-    // read.  sc0: measured 3-7 % faster than the default policy.  M0 (the
-    // copy's LDS base) is set by the same statement; nothing else in these
-    // kernels uses M0 (clang warns that the clobber names a reserved register).
-    // The base is read back from lane 0: it is uniform, and the SGPR operand
-    // then needs no proof of it from the compiler.
+    // The copies (lds_copy16), with the explicit waits below.  sc0: measured
+    // 3-7 % faster than the default policy.  The base is read back from lane
+    // 0: it is uniform, and the SGPR operand then needs no proof of it from
+    // the compiler.
     const uint64_t sv = (uint64_t)(uintptr_t)(src + s0 * G16_BK);
     const uint64_t bw = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(sv >> 32)) << 32) |
                         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)sv);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
     auto copy1 = [&](int st, _Float16 *S, int i) {
         const uint64_t base = bw + (uint64_t)st * (2 * G16_BK);
         const uint32_t dst = (uint32_t)(uintptr_t)&S[16 * (8 * wave + i) * G16_BK];
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 sc0" ::"v"(off[i]), "s"(base), "s"(dst)
-                     : "memory", "m0");
+        lds_copy16<true>(off[i], base, dst);
     };
-#pragma clang diagnostic pop
 
     g16_acc acc[8][8];
 #pragma unroll
@@ -381,15 +373,11 @@ __device__ static inline void gemm16_w8_body(const Gemm16Args &a) {
     const uint64_t sv = (uint64_t)(uintptr_t)(src + s0 * G16_BK);
     const uint64_t bw = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(sv >> 32)) << 32) |
                         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)sv);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
     auto copy1 = [&](int st, _Float16 *S, int i) {
         const uint64_t base = bw + (uint64_t)st * (2 * G16_BK);
         const uint32_t dst = (uint32_t)(uintptr_t)&S[16 * (4 * wave + i) * G16_BK];
-        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 sc0" ::"v"(off[i]), "s"(base), "s"(dst)
-                     : "memory", "m0");
+        lds_copy16<true>(off[i], base, dst);
     };
-#pragma clang diagnostic pop
 
     g16_acc acc[8][4];
 #pragma unroll

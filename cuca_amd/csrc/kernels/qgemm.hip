@@ -229,9 +229,7 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     const uint32_t woff = (uint32_t)r * (uint32_t)a.row_bytes + 16u * (uint32_t)u;
     // The copies: wave w fills LDS rows w TM / 4 .., four rows of 256 bytes an
     // instruction (lane L: row L / 16 of them, unit L % 16, from source unit
-    // (L % 16) ^ (row & 7)).  Issued from inline assembly with the waits
-    // written out: the compiler cannot tell the two buffers apart behind an
-    // LDS DMA and would wait for the copies before any LDS read.
+    // (L % 16) ^ (row & 7)).  The waits are written out below.
     uint32_t off[2];
 #pragma unroll
     for (int i = 0; i < 2; i++)
@@ -240,18 +238,14 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     const uint64_t xb = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(xv >> 32)) << 32) |
                         (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)xv);
     const uint64_t x4 = 8 * (uint64_t)a.kp; // bytes of four rows
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
     auto copy = [&](int kc, int buf) {
 #pragma unroll
         for (int i = 0; i < TM / 16; i++) {
             const uint64_t src = xb + i * x4 + (uint64_t)kc * (2 * QG_KC);
             const uint32_t dst = (uint32_t)(uintptr_t)&xs[(buf * TM + wave * (TM / 4) + 4 * i) * QG_KC];
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off[i & 1]), "s"(src), "s"(dst)
-                         : "memory", "m0");
+            lds_copy16(off[i & 1], src, dst);
         }
     };
-#pragma clang diagnostic pop
     qg_acc acc[4][NT];
 #pragma unroll
     for (int i = 0; i < 4; i++)

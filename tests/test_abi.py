@@ -44,6 +44,29 @@ def test_code_object_is_gfx950_only_and_lists_every_kernel():
     assert sizes and max(sizes) == 0
 
 
+def test_a_wait_state_stands_between_a_write_of_m0_and_the_lds_copy_that_reads_it():
+    """A copy straight into LDS takes its LDS base from M0, and gfx9 wants one
+    instruction between a scalar write of M0 and the copy.  The compiler's own
+    hazard pass does not see an M0 write inside an asm string, so this reads
+    the built code."""
+    dis = subprocess.Popen([os.path.join(build.ROCM, "llvm/bin/llvm-objdump"), "-d", "--no-show-raw-insn",
+                            build.CODE_OBJECT], stdout=subprocess.PIPE, text=True)
+    copies, bad, last, symbol = 0, [], "", ""
+    for line in dis.stdout:
+        if line[0] != "\t":
+            symbol = line.strip()
+            continue
+        ins = line.split("//")[0].strip()
+        op = ins.split(None, 1)[0]
+        if "_load_lds" in op or (op.startswith("buffer_load") and re.search(r"\blds\b", ins)):
+            copies += 1
+            if re.match(r"\S+ m0\b", last):
+                bad.append(f"{symbol} {last}; {ins}")
+        last = ins
+    assert dis.wait() == 0
+    assert copies > 0 and not bad, (copies, bad[:4])
+
+
 @pytest.mark.parametrize("spec", [
     dict(n_dims=128, base=1e6, positions=64),
     dict(n_dims=128, base=5e5, positions=8192),
