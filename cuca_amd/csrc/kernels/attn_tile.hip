@@ -325,7 +325,10 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
             acc[d][i] = zero ? 0.0f : __builtin_fmaf(__builtin_fmaf(-o, l, acc[d][i]), rl, o);
             fin = fin && __builtin_fabsf(acc[d][i]) < __builtin_huge_valf();
         }
-    fin = fin && __shfl_xor((int)fin, 32);
+    // both halves of a row agree (the exchange outside the &&: behind it only
+    // lanes whose own is true would ask, and the compiler takes the answer as known)
+    const int fin_other = __shfl_xor((int)fin, 32);
+    fin = fin && fin_other;
     // A weight of zero times an infinite or NaN value outside the row's range
     // is a NaN that the row must not see: such a row (its weights are finite)
     // is done again position by position.

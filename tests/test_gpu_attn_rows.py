@@ -66,7 +66,7 @@ def run_rows(ctx, q, pk, pv, table, ranges, n_head, scale, q_ld=None):
     qpad[:, :n_head * d] = q.reshape(rows, -1)
     dq, dk, dv = ctx.array(qpad), ctx.array(pk), ctx.array(pv)
     dt, dr = ctx.array(table.astype(np.uint32)), ctx.array(ranges.astype(np.int32))
-    out = ctx.empty((rows, n_head, d), q.dtype)
+    out = ctx.array(np.full((rows, n_head, d), 7.0, q.dtype))  # (what is not written shows)
     ctx.attend_rows(dq.ptr, q_ld, dk.ptr, dv.ptr, n_blocks, dt.ptr, len(table), dr.ptr, rows, n_head, n_kv, d,
                     scale, out.ptr, n_head * d, hip.dtype_code(q.dtype))
     ctx.check_device()
@@ -213,6 +213,28 @@ def test_f16_tiles_at_their_edges(ctx, nq, nk, d, t, start, scale):
         got = run_rows(ctx, q, pk, bad, table, ranges, nq, scale)
         assert_close(got[:-1], all_rows[:-1], floor=floor_of(table, ranges[:-1], pv, nq), what="rows before it")
         assert not np.isfinite(got[-1].astype(np.float32)).any()
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("col", [1, 6])  # a column of each half-wave's: col % 8 below and from 4
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_f16_one_value_that_is_not_finite(ctx, d, col, value):
+    """One column of the last position's value in one KV head is not finite:
+    the rows before it, whose tile holds it at weight zero, and every other
+    column of the last row come out whole, the last row's column as it is."""
+    rng = np.random.default_rng(d + col)
+    nq, nk, t, start, n_blocks = 4, 2, 45, 20, 8
+    pk, pv = (rng.standard_normal((n_blocks, nk, 16, d)).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((t, nq, d)).astype(np.float16)
+    table, ranges = chunk(rng, t, start, n_blocks, n_blocks)
+    want = want_rows(q, pk, pv, table, ranges, 0.1)
+    bad, last = pv.copy(), t + start - 1
+    bad[table[last // 16], 1, last % 16, col] = value
+    got = run_rows(ctx, q, pk, bad, table, ranges, nq, 0.1)
+    at = got[-1, 2:, col].copy()  # KV head 1's query heads
+    assert not np.isfinite(at.astype(np.float32)).any()
+    got[-1, 2:, col] = want[-1, 2:, col]
+    assert_close(got, want, floor=floor_of(table, ranges, pv, nq), what=f"column {col} of {d}")
 
 
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
