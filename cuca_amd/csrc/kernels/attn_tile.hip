@@ -19,10 +19,15 @@
 //    key mod 16, V: pairs of pieces by key mod 4), in the source addresses of
 //    the copies; no bank conflicts (SQ_LDS_BANK_CONFLICT 0).
 //  * A weight enters the value product as two f16 parts, hi = f16(p) and lo =
-//    f16(p - hi), 22 bits of it, into one accumulator: weights are held times
-//    2^7, at most 2^15 (the running maximum is raised only by steps above 2^8,
-//    so most tiles skip the accumulators' rescale), so lo keeps its bits, down
-//    to 2^-32 of a row's largest weight.
+//    f16(p - hi), 22 bits of it.  Weights are held times 2^12, at most 2^15 (the
+//    running maximum is raised only by steps above 2^3, so most tiles skip the
+//    accumulators' rescale), so lo keeps its bits for weights down to 2^-15 of
+//    the largest, and 2^-37 of it below (times 2^7 after steps of 2^8: down to
+//    2^-10).
+//  * A tile's value product is summed from zero, lo and hi in one chain, and
+//    then added: the accumulators round once every 64 keys.  (The chain run in
+//    the accumulators themselves rounds eight times; values that cancel then lost
+//    1.4 times what one rounding every 16 keys loses, and 3 times what this does.)
 //  * The next tile's score products issue between this one's exponentials and
 //    conversions, two matrix instructions and eight scores' arithmetic a step.
 //
@@ -31,10 +36,10 @@
 // wave alternates between them (a value product has no arithmetic to hide
 // behind) and waits at the tile's barrier a fifth of the time.  MI355X, us,
 // before (16-key blocks, 16x16x16 products, a row tile of 16) -> after: causal
-// 4096 rows of 32 heads over 8 of 128: 502 -> 212; with a window of 1024 238
-// -> 119; 2048 rows of 16 heads of 256: 205 -> 117; 8 rows after 4096 keys,
-// 32 heads over 4: 277 -> 111 (one workgroup a head group: latency).  Without
-// the interleaving 255 for 250 at 4096 rows, 68 for 63 at 2048 of 16 heads.
+// 4096 rows of 32 heads over 8 of 128: 505 -> 227 (218 with the chain in the
+// accumulators); with a window of 256 71 -> 50; 2048 rows of 16 heads over 8 of
+// 256: 197 -> 110; 8 rows after 4096 keys, 32 heads over 4: 279 -> 108 (one
+// workgroup a head group: latency).
 #include "common.h"
 
 #pragma clang fp contract(off)
@@ -239,7 +244,7 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
 #pragma unroll
                     for (int i = 0; i < 16; i++) bm = fmaxf(bm, st[k][i]);
                 bm = fmaxf(bm, __shfl_xor(bm, 32)) * scale2;
-                const bool up = bm > m + 8.0f;
+                const bool up = bm > m + 3.0f;
                 if (__ballot(up)) {
                     const float corr = up ? __builtin_amdgcn_exp2f(m - bm) : 1.0f;
                     l *= corr;
@@ -248,7 +253,7 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
                     m = up ? bm : m;
                 }
                 // the next tile's scores on the matrix cores, this one's weights beside them
-                const float m7 = 7.0f - m;
+                const float m12 = 12.0f - m;
                 uint32_t ph[NK][8], pl[NK][8];
                 at_f16v sn[NK];
                 {
@@ -271,8 +276,8 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
 #pragma unroll
                         for (int n = j * PAIRS; n < (j + 1) * PAIRS && n < 8 * NK; n++) {
                             const int k = n >> 3, i = 2 * (n & 7);
-                            const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i], scale2, m7));
-                            const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i + 1], scale2, m7));
+                            const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i], scale2, m12));
+                            const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i + 1], scale2, m12));
                             s0 += e0;
                             s1 += e1;
                             const at_h2 p = __builtin_convertvector(at_f2{e0, e1}, at_h2);
@@ -285,24 +290,37 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
                     l += s0 + s1;
                 }
                 const unsigned char *vb = kv[t & 1][1];
+                typedef __attribute__((address_space(3))) at_s4 *lds4;
+                auto value = [&](int d, int s) { // columns 32 d .. of keys 16 s .. 16 s + 15
+                    const at_s4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vb + va[d] + 16 * s * RB));
+                    const at_s4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vb + va[d] + (16 * s + 8) * RB));
+                    return __builtin_bit_cast(at_h8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+                };
+                // a slice of 32 columns at a time from zero, added to its accumulators
+                // beside the next slice's products
+                constexpr int NS = KT / 16;
+                at_f16v sum[2];
+                at_h8 v[2];
+                v[0] = value(0, 0);
 #pragma unroll
-                for (int s = 0; s < KT / 16; s++) {
-                    typedef __attribute__((address_space(3))) at_s4 *lds4;
-                    at_h8 v[ND];
+                for (int d = 0; d < ND; d++)
 #pragma unroll
-                    for (int d = 0; d < ND; d++) {
-                        const at_s4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vb + va[d] + 16 * s * RB));
-                        const at_s4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vb + va[d] + (16 * s + 8) * RB));
-                        v[d] = __builtin_bit_cast(at_h8, __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7));
+                    for (int s = 0; s < NS; s++) {
+                        const int n = d * NS + s;
+                        if (n + 1 < ND * NS) v[(n + 1) & 1] = value((n + 1) / NS, (n + 1) % NS);
+                        const uint32_t *hp = &ph[s >> 1][4 * (s & 1)], *lp = &pl[s >> 1][4 * (s & 1)];
+                        const at_h8 bh = __builtin_bit_cast(at_h8, u32x4{hp[0], hp[1], hp[2], hp[3]});
+                        const at_h8 bl = __builtin_bit_cast(at_h8, u32x4{lp[0], lp[1], lp[2], lp[3]});
+                        sum[d & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n & 1], bl, s ? sum[d & 1] : at_f16v{}, 0, 0, 0);
+                        sum[d & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n & 1], bh, sum[d & 1], 0, 0, 0);
+                        if (d && s) { // (not behind the first: the slice's sums are not there yet)
+#pragma unroll
+                            for (int i = 16 * (s - 1) / (NS - 1); i < 16 * s / (NS - 1); i++)
+                                acc[d - 1][i] += sum[(d - 1) & 1][i];
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    const uint32_t *hp = &ph[s >> 1][4 * (s & 1)], *lp = &pl[s >> 1][4 * (s & 1)];
-                    const at_h8 bh = __builtin_bit_cast(at_h8, u32x4{hp[0], hp[1], hp[2], hp[3]});
-                    const at_h8 bl = __builtin_bit_cast(at_h8, u32x4{lp[0], lp[1], lp[2], lp[3]});
-#pragma unroll
-                    for (int d = 0; d < ND; d++) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[d], bh, acc[d], 0, 0, 0);
-#pragma unroll
-                    for (int d = 0; d < ND; d++) acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[d], bl, acc[d], 0, 0, 0);
-                }
+                acc[ND - 1] += sum[(ND - 1) & 1];
 #pragma unroll
                 for (int k = 0; k < NK; k++) st[k] = sn[k];
             }

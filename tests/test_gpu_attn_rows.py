@@ -237,6 +237,61 @@ def test_f16_one_value_that_is_not_finite(ctx, d, col, value):
     assert_close(got, want, floor=floor_of(table, ranges, pv, nq), what=f"column {col} of {d}")
 
 
+def test_f16_small_weights_keep_their_bits(ctx):
+    """Two keys of nearly equal weights 2^-9 to 2^-14 of the row's largest
+    and opposite values beside one of weight one and value zero: the row is
+    their difference, 2^-10 of either, so the bits of the weights below f16's
+    show.  The bound: 22 bits of a weight (two f16 parts), the exponential (one
+    unit of f32), four roundings of the sums, and the output's own rounding."""
+    nk, d, t = 6, 64, 40
+    pk, pv = np.zeros((1, nk, 16, d), np.float16), np.zeros((1, nk, 16, d), np.float16)
+    for e in range(nk):  # score: -(9 + e) and that less q[1] / 1024, in units of log 2
+        pk[0, e, 1, 0] = pk[0, e, 2, 0] = -(9.0 + e)
+        pk[0, e, 2, 1] = -2.0 ** -10
+        pv[0, e, 1] = 16384.0 + 128.0 * np.arange(d)
+        pv[0, e, 2] = -pv[0, e, 1]
+    q = np.zeros((t, nk, d), np.float16)
+    q[:, :, 0], q[:, :, 1] = 1.0, (1.0 + np.arange(t) / 64.0)[:, None]
+    scale = np.float32(np.log(2.0))
+    got = run_rows(ctx, q, pk, pv, np.zeros(1, np.uint32), np.tile(np.array([[0, 3]], np.int32), (t, 1)), nk, scale)
+    w = np.exp(np.einsum("thd,hkd->thk", q.astype(np.float64), pk[0, :, :3].astype(np.float64)) * np.float64(scale))
+    v = pv[0, :, :3].astype(np.float64)
+    want = np.einsum("thk,hkd->thd", w, v) / w.sum(-1)[..., None]
+    mass = np.einsum("thk,hkd->thd", w, np.abs(v)) / w.sum(-1)[..., None]
+    bar = mass * (2.0 ** -22 + 2.0 ** -23 + 4 * 2.0 ** -24) + 2.0 ** -11 * np.abs(want)
+    err = np.abs(got.astype(np.float64) - want)
+    assert np.all(err <= bar), float(np.max(err / bar))
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("half", [512, 2048])
+def test_f16_sums_round_no_more_than_once_every_16_keys(ctx, d, half):
+    """Values that cancel: the second half of the keys is the first again with
+    its values negated, so a row is what its f32 sums lost on the way.  The
+    bar is that of sums rounded to nearest once every 16 keys (uniform errors
+    of a unit in the last place of the partial sums, known in 64 bits, over
+    the outputs' root mean square)."""
+    rng = np.random.default_rng(d + half)
+    nk, t, nb = 2, 16, 2 * half // 16
+    k1, v1 = rng.standard_normal((nk, half, d)), 1024.0 * rng.standard_normal((nk, half, d))
+    k, v = (np.concatenate(x, 1).astype(np.float16) for x in ((k1, k1), (v1, -v1)))
+    pk, pv = (np.ascontiguousarray(x.reshape(nk, nb, 16, d).transpose(1, 0, 2, 3)) for x in (k, v))
+    q, scale = rng.standard_normal((t, nk, d)).astype(np.float16), 1.0 / np.sqrt(d)
+    got = run_rows(ctx, q, pk, pv, np.arange(nb, dtype=np.uint32), np.tile(np.array([[0, 2 * half]], np.int32), (t, 1)),
+                   nk, scale)
+    s = np.einsum("thd,hkd->thk", q.astype(np.float64), k.astype(np.float64)) * scale
+    w = np.exp(s - s.max(-1, keepdims=True))
+    var = np.zeros((t, nk, d))
+    acc = np.zeros((t, nk, d))
+    for b in range(nb):
+        at = slice(16 * b, 16 * b + 16)
+        acc += np.einsum("thk,hkd->thd", w[..., at], v[:, at].astype(np.float64))
+        var += 2.0 ** (2 * (np.floor(np.log2(np.abs(acc) + 1e-30)) - 23)) / 12
+    bar = np.sqrt((var / w.sum(-1)[..., None] ** 2).mean())
+    rms = np.sqrt((got.astype(np.float64) ** 2).mean())
+    assert rms <= bar, (rms, bar)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
 @pytest.mark.parametrize("nh,d,vw,t", [(16, 576, 512, 21), (4, 80, 64, 33)])
 def test_latent_rows(ctx, dtype, nh, d, vw, t):
