@@ -11,14 +11,15 @@
 // all the tile's pairs; a tile of fewer than four pairs runs a body of its own
 // (MJ), so that no chain is computed for a pair that is not there.  A task's
 // sums go to LDS and a chunk of QMS_MOE_NT tasks is written after its stream,
-// so that the ring's waits count its own loads only.  The splits are a
-// multiple of eight: a split of all an expert's tiles meets in one XCD's L2.
+// so that the ring's waits count its own loads only.  Where the splits are a
+// multiple of eight, a split of all an expert's tiles meets in one XCD's L2.
 //
 // What bounds it: the vector unit's issue rate (Q4_0 and Q8_0 take the same
 // time), as qms.hip.  Measured on MI355X, 128 experts of 768 over 2048, top 8,
-// Zipf routing, f32, up + down + sum: 32 tokens 145 -> 115 us against the kernel
-// before it (tiles of one to four pairs by the mean, every tile's chains
-// computed for all of them, dw * dx and the pairs' bias through LDS).
+// Zipf routing, f32 Q4_0, up + down, 2 / 4 / 8 / 16 / 32 / 64 tokens: 16 / 24 / 37
+// / 65 / 106 / 176 us, against the kernel before it (tiles of one to four pairs
+// by the mean, every tile's chains computed for all of them, dw * dx and the
+// pairs' bias through LDS) 25 / 27 / 47 / 69 / 139 / 342.
 #include "common.h"
 
 #define QMS_MOE_WAVES 4

@@ -2652,21 +2652,33 @@ static cuca_status moe_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
     auto tiles = [&](int64_t t) { return (max_pairs + (t - 1) * std::min<int64_t>(n_experts, max_pairs)) / t; };
     // qms_moe.hip, a workgroup per (tile, split of the expert's rows), from
     // two tokens' pairs up (16 pairs over 128 experts); a single token's
-    // pairs keep the one-pass kernel.  Tiles of four pairs where two such
-    // workgroups fit a compute unit's LDS, of fewer (for longer rows) where
-    // the experts hold no more on average; otherwise the one-pass kernel
+    // pairs keep the one-pass kernel, and so does down where its waves (a task
+    // of eight rows each) are fewer than six a compute unit: with no other wave
+    // to hide behind, a wave of four rows is done sooner (2048 x 8192, 2 / 4 / 6
+    // pairs: 9.9 / 12.0 / 14.8 us against 14.1 / 14.1 / 18.2).  Tiles of one pair
+    // where the experts hold no more on average, else of four where two such
+    // workgroups fit a compute unit's LDS, of fewer for longer rows (as many as
+    // the experts hold on average); otherwise the one-pass kernel
     auto lds = [&](int64_t t) { return qms_lds(t, ng * g) + (size_t)t * 4 * 16 * 8 * 4; }; // QMS_MOE_LDS_BYTES
-    const int64_t tr = lds(4) <= (80u << 10) ? 4 : mt <= 2 && lds(2) <= (80u << 10) ? 2
-                                             : mt == 1 && lds(1) <= (80u << 10) ? 1 : 0;
-    if (16 * max_pairs > n_experts && tr && packed < (1ll << 31)) {
-        const int64_t nt = tiles(tr), ntask = up ? (n + 3) / 4 : (n + 7) / 8;
-        // eight workgroups a compute unit by the tile bound (about half of it
-        // is there at 32 tokens; at 2 / 4 / 8 / 16: 127, 127, 115, 125 us), in
-        // eights: blockIdx % 8 is the XCD, so a split of all an expert's
-        // tiles reads its rows from one L2
-        int64_t splits = (((int64_t)ctx->cu_count * 8 + nt - 1) / nt + 7) / 8 * 8;
+    constexpr size_t half = 80u << 10;
+    const int64_t tr = mean <= 1.0 && lds(1) <= half ? 1 : lds(4) <= half ? 4
+                       : mt <= 2 && lds(2) <= half ? 2 : mt == 1 && lds(1) <= half ? 1 : 0;
+    const int64_t ntask = up ? (n + 3) / 4 : (n + 7) / 8;
+    const bool enough = up || max_pairs * ntask > 6 * (int64_t)ctx->cu_count;
+    if (16 * max_pairs > n_experts && tr && enough && packed < (1ll << 31)) {
+        const int64_t nt = tiles(tr);
+        // Workgroups by the tile bound.  Tiles of one pair are all there: what
+        // the compute units hold at once, four each (128 experts of 768 over 2048,
+        // top 8, 4 tokens, up / down: one task a wave in a second round 15.4 / 12.0
+        // us, two tasks in one 13.4 / 10.1).  Of larger tiles about half the bound
+        // is there: eight each (32 tokens, at 2 / 4 / 8 / 16: 127, 127, 115, 125 us).
+        // Eights of splits where they allow it: blockIdx % 8 is the XCD, so a split
+        // of all an expert's tiles reads its rows from one L2.
+        const int64_t wgs = (int64_t)ctx->cu_count * (tr == 1 ? 4 : 8);
+        int64_t splits = tr == 1 ? std::max<int64_t>(8, wgs / nt / 8 * 8) : ((wgs + nt - 1) / nt + 7) / 8 * 8;
         splits = std::min<int64_t>(splits, (ntask + 3) / 4);
         const int64_t tps = ((ntask + splits - 1) / splits + 3) / 4 * 4;
+        splits = (ntask + tps - 1) / tps; // (none without rows: they would take the place of others)
         if (tps * splits > 0x7fffffffll || nt * splits > 0x7fffffffll)
             return fail(ctx, CUCA_UNSUPPORTED, "moe: grid too large");
         // [dtype][format][down, up]

@@ -139,7 +139,11 @@ def test_moe_layer(ctx, qtype, dtype, act, t, n_experts, n_used, n_embd, ff):
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
 @pytest.mark.parametrize("counts,rows,k", [([1, 0, 2, 3, 4, 5, 7, 9], 37, 544), ([3, 4], 4, 32),
                                            ([1, 2, 3, 4] * 64, 1029, 96), ([3, 0, 1, 2, 0, 1, 4, 0], 29, 12288),
-                                           ([3, 0, 1, 2, 0, 1, 4, 0], 13, 20480)])
+                                           ([3, 0, 1, 2, 0, 1, 4, 0], 13, 20480),
+                                           # down's rows enough for its decode kernel, and tiles of one pair
+                                           ([1, 0, 2, 3, 4, 5, 7, 9], 405, 544), ([1, 0, 1, 2, 0, 1, 0, 3], 1541, 288),
+                                           ([3, 0, 1, 2, 0, 1, 4, 0], 1125, 12288),
+                                           ([3, 0, 1, 2, 0, 1, 4, 0], 1125, 20480)])
 def test_decode_kernel_tiles(ctx, qtype, dtype, counts, rows, k):
     rng = np.random.default_rng(rows + k)
     npd = np.float16 if dtype == "f16" else np.float32
@@ -173,6 +177,26 @@ def test_decode_kernel_tiles(ctx, qtype, dtype, counts, rows, k):
         assert_close(got_h[lo:hi], wh.astype(npd), what=f"moe_up expert {e}")
         y = O.qmm(down, QT[qtype], rows, k, x[lo:hi].astype(np.float32))
         assert_bits_equal(got_s[lo:hi], (y * wt[lo:hi, None]).astype(np.float32), f"moe_down expert {e}")
+
+
+@pytest.mark.parametrize("pairs,up,down", [(2, "cuca_qms_moe_up", "cuca_moe_down"), (6, "cuca_qms_moe_up", "cuca_moe_down"),
+                                           (8, "cuca_qms_moe_up", "cuca_qms_moe_down")])
+def test_down_of_few_pairs_keeps_the_one_pass_kernel(ctx, pairs, up, down):
+    """2048 rows are 256 tasks of eight a pair: the decode kernel takes down
+    from more than six waves a compute unit (1536) on."""
+    E, n, k = 8, 2048, 64
+    rng = np.random.default_rng(pairs)
+    one = (hip.qweight_bytes(QT["q4_0"], n, k) + 15) // 16 * 16
+    w, x = ctx.array(np.zeros(E * one, np.uint8)), ctx.array(rng.standard_normal((pairs, k)).astype(np.float32))
+    off = ctx.array(np.minimum(np.arange(E + 1), pairs).astype(np.int32))
+    tok, wt = ctx.array(np.arange(pairs, dtype=np.int32)), ctx.array(np.ones(pairs, np.float32))
+    out = ctx.empty((pairs, n), np.float32)
+    ctx.profile_start(4)
+    ctx.moe_up(w.ptr, w.ptr, one, QT["q4_0"], n, k, E, x.ptr, k, pairs, off.ptr, tok.ptr, pairs, hip.ACT_SILU, 0.0,
+               out.ptr, n, hip.F32)
+    ctx.moe_down(w.ptr, one, QT["q4_0"], n, k, E, x.ptr, k, off.ptr, wt.ptr, pairs, out.ptr, n, hip.F32)
+    names = [name for name, _ in ctx.profile_stop()]
+    assert len(names) == 2 and names[0].startswith(up) and names[1].startswith(down), names
 
 
 def test_moe_sum_adds_in_the_given_order(ctx):
