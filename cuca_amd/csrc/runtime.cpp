@@ -1633,14 +1633,18 @@ static cuca_status qmm_common(cuca_hip_ctx *ctx, const void *w, const void *w_up
     if (!al16(x) || ((size_t)ldx * es) % 16 != 0)
         return fail(ctx, CUCA_INVALID_ARG, "qmm: activation rows must start 16-byte aligned");
     const int64_t nb = k / 32, ng = (nb + g - 1) / g;
-    // one or two rows of a tall matrix whose tile fits the LDS and that the
-    // one-row and several-row kernels do not take (2 GiB and more): the decode
-    // GEMV stream, each workgroup quantising the rows itself.  Below that the
-    // others are faster (MI355X, the 128256 x 4096 LM head, Q8_0 / Q4_0: one
-    // row 101-103 -> 88-89 us / 59-60 -> 51 us, two rows 131 -> 109 us / 100
-    // -> 88 us)
+    // One or two rows of a tall matrix whose tile fits the LDS: the decode
+    // GEMV stream, each workgroup quantising the rows itself, where the one-row
+    // and several-row kernels do not take the matrix (2 GiB and more), and for
+    // two rows where its waves, which carry on from task to task, beat the
+    // several-row kernel's workgroups, which end after 64 weight rows: many of
+    // these and short rows.  MI355X, us, several rows / stream, f32: Q8_0 400000 x
+    // 256 51.7 / 31.3, 256000 x 1536 91.6 / 84.3, x 2560 144 / 135, x 3584 190 / 191,
+    // x 4096 209 / 255; 81920 x 1024 23.6 / 26.3; Q4_0 (whose rows are half the
+    // bytes) 256000 x 512 34.5 / 29.0, x 1024 48.7 / 49.2
+    const bool stream2 = !glu && rows >= 98304 && k <= (ggml_type == CUCA_GGML_Q8_0 ? 2560 : 512);
     const bool qmv = m <= 2 && qmv_wins(ctx, rows) && qmv_fits(m, ng * g, g) &&
-                     !(m == 1 ? qmd_fits(m, k, ng, g, rows, ng * gb) : rows * ng * gb < (1ll << 31));
+                     !(m == 1 ? qmd_fits(m, k, ng, g, rows, ng * gb) : rows * ng * gb < (1ll << 31) && !stream2);
     if (qmv) {
         if (rn && (st = norm_in_launch(ctx, *rn, m, k, dtype)) != CUCA_OK) return st;
         return qmv_launch(ctx, 3, w, w_up, ggml_type, n, k, nullptr, 0, nullptr, x, ldx, m, rows, glu, clamp, out,

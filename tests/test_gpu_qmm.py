@@ -335,6 +335,18 @@ def test_decode_gemv_streams_chunks_of_tasks(ctx, qtype):
     assert_bits_equal(out.numpy(), want, "streamed chunks, quantised rows")
 
 
+@pytest.mark.parametrize("qtype,n,k,kernel", [
+    ("q8_0", 98304, 64, "cuca_qmvx_q8_0_m2"), ("q8_0", 98300, 64, "cuca_qms"), ("q8_0", 98304, 2560, "cuca_qmvx_q8_0_m2"),
+    ("q8_0", 98304, 2592, "cuca_qms"), ("q4_0", 98304, 512, "cuca_qmvx_q4_0_m2"), ("q4_0", 98304, 544, "cuca_qms")])
+def test_two_rows_of_a_tall_matrix_of_short_rows_are_streamed(ctx, qtype, n, k, kernel):
+    w = ctx.empty((hip.qweight_bytes(QT[qtype], n, k),), np.uint8)
+    x, out = ctx.array(np.zeros((2, k), np.float32)), ctx.empty((2, n), np.float32)
+    ctx.profile_start(4)
+    ctx.qmm(w.ptr, QT[qtype], n, k, x.ptr, k, 2, n, out.ptr, n, hip.F32)
+    names = [name for name, _ in ctx.profile_stop()]
+    assert len(names) == 1 and names[0].startswith(kernel), names
+
+
 # ---------------------------------------------------------------------------
 # the Q|K|V projection with RoPE and the paged K/V store in its epilogue
 # (cuca_hip_qmm_rope_store_kv): the bits of qmm followed by rope_store_kv
