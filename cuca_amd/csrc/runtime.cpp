@@ -1570,15 +1570,27 @@ static bool qms_launch(cuca_hip_ctx *ctx, int mode, int glu, uint32_t ggml_type,
     // against 8.5 us; down 19.8 against 22.2)
     if (m == 2 && !wide) return false;
     a.js = wide ? 1 : tr > 2 ? 2 : 1;
-    if (!wide && tr == 3 && qms_lds(4, nbp) > kQmsLds) { a.js = 1; tr = 2; }
+    if (!wide && qms_lds(4, nbp) > kQmsLds) {
+        // rows so long that a workgroup of 16 weight rows holds two of them and a
+        // compute unit one workgroup: a round of them streams the weight at two
+        // rows each.  Past one round the chunked kernel's tiles of four are faster
+        // (5376 x 21504 Q4_0, 4 / 8 rows: 74 / 112 us against 91 / 178; 3584 x
+        // 21504, 12 rows: 0.63 of the time; 2048 x 21504 at 4 rows, one round: 50
+        // against 30)
+        a.js = 1;
+        tr = 2;
+        if (m <= 16 && (a.rows + 15) / 16 * ((m + 1) / 2) > cus) return false;
+    }
     a.tile_rows = (int32_t)tr;
     a.ntile = (int32_t)((m + tr - 1) / tr);
     a.gelu = glu == 2;
-    // 4 waves a workgroup where 8 leave compute units idle (gate and up of
-    // 3072 x 1024 at four rows: 7.8 -> 6.5 us); 16 where the rows fill a
+    // 4 waves a workgroup where 8 leave compute units idle and 4 run in one round
+    // (gate and up of 3072 x 1024 at four rows: 7.8 -> 6.5 us); 16 where the rows fill a
     // compute unit's LDS and workgroups of 8 would take turns (4096 x 14336 at
     // eight rows: 55.5 -> 40.3 us, the chunked kernel 50)
-    int waves = wide ? (glu && (a.rows + 31) / 32 * a.ntile < cus ? 4 : 8) : 4 * a.js;
+    const bool four = glu && (a.rows + 31) / 32 * a.ntile < cus &&
+                      (a.rows + 15) / 16 * a.ntile <= cus * (int64_t)(kQmsLds / qms_lds(tr, nbp));
+    int waves = wide ? (four ? 4 : 8) : 4 * a.js;
     if (!wide && a.js == 2 && qms_lds(4, nbp) > kQmsLds / 2 && (a.rows + 15) / 16 * a.ntile > cus) waves = 16;
     const int64_t per_wg = waves / a.js * (wide && !glu ? 8 : 4); // weight rows (of each matrix) a workgroup
     a.nrb = (int32_t)((a.rows + per_wg - 1) / per_wg);

@@ -335,6 +335,18 @@ def test_decode_gemv_streams_chunks_of_tasks(ctx, qtype):
     assert_bits_equal(out.numpy(), want, "streamed chunks, quantised rows")
 
 
+@pytest.mark.parametrize("n,k,m,kernel", [
+    (2048, 18432, 4, "cuca_qms_f32_q4_0_w1"), (2064, 18432, 4, "cuca_qmm_f32_q4_0_m4"),
+    (2064, 18432, 16, "cuca_qmm_f32_q4_0_m4"), (2064, 18432, 17, "cuca_qms_f32_q4_0_w1"), (2064, 17408, 16, "cuca_qms_f32_q4_0_w1")])
+def test_rows_past_the_lds_take_the_chunked_kernel_from_a_second_round_on(ctx, n, k, m, kernel):
+    w = ctx.empty((hip.qweight_bytes(QT["q4_0"], n, k),), np.uint8)
+    x, out = ctx.array(np.zeros((m, k), np.float32)), ctx.empty((m, n), np.float32)
+    ctx.profile_start(4)
+    ctx.qmm(w.ptr, QT["q4_0"], n, k, x.ptr, k, m, n, out.ptr, n, hip.F32)
+    names = [name for name, _ in ctx.profile_stop()]
+    assert len(names) == 1 and names[0].startswith(kernel), names
+
+
 @pytest.mark.parametrize("qtype,n,k,kernel", [
     ("q8_0", 98304, 64, "cuca_qmvx_q8_0_m2"), ("q8_0", 98300, 64, "cuca_qms"), ("q8_0", 98304, 2560, "cuca_qmvx_q8_0_m2"),
     ("q8_0", 98304, 2592, "cuca_qms"), ("q4_0", 98304, 512, "cuca_qmvx_q4_0_m2"), ("q4_0", 98304, 544, "cuca_qms")])
