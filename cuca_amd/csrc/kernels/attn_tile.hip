@@ -29,7 +29,8 @@
 //    the accumulators themselves rounds eight times; values that cancel then lost
 //    1.4 times what one rounding every 16 keys loses, and 3 times what this does.)
 //  * The next tile's score products issue between this one's exponentials and
-//    conversions, two matrix instructions and eight scores' arithmetic a step.
+//    conversions, two matrix instructions and eight scores' arithmetic a step; a
+//    wave's last tile has none, and weighs only the 16 keys its ranges reach.
 //
 // What bounds it: the matrix cores are busy 57 % and the vector unit 48 % of
 // the time a compute unit works, at two waves a SIMD and about 1.9 GHz; each
@@ -96,10 +97,10 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
     int ilo = valid ? lo : 0, ihi = valid ? hi : 0x7fffffff;
 #pragma unroll
     for (int off = 1; off < 32; off <<= 1) {
-        wlo = min(wlo, __shfl_xor(wlo, off));
-        whi = max(whi, __shfl_xor(whi, off));
-        ilo = max(ilo, __shfl_xor(ilo, off));
-        ihi = min(ihi, __shfl_xor(ihi, off));
+        wlo = min(wlo, (int)xor_partner_bits((uint32_t)wlo, off));
+        whi = max(whi, (int)xor_partner_bits((uint32_t)whi, off));
+        ilo = max(ilo, (int)xor_partner_bits((uint32_t)ilo, off));
+        ihi = min(ihi, (int)xor_partner_bits((uint32_t)ihi, off));
     }
     wlo = __builtin_amdgcn_readfirstlane(wlo);
     whi = __builtin_amdgcn_readfirstlane(whi);
@@ -243,7 +244,7 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
                 for (int k = 0; k < NK; k++)
 #pragma unroll
                     for (int i = 0; i < 16; i++) bm = fmaxf(bm, st[k][i]);
-                bm = fmaxf(bm, __shfl_xor(bm, 32)) * scale2;
+                bm = fmaxf(bm, xor_partner(bm, 32)) * scale2;
                 const bool up = bm > m + 3.0f;
                 if (__ballot(up)) {
                     const float corr = up ? __builtin_amdgcn_exp2f(m - bm) : 1.0f;
@@ -252,18 +253,29 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
                     for (int d = 0; d < ND; d++) acc[d] *= corr;
                     m = up ? bm : m;
                 }
-                // the next tile's scores on the matrix cores, this one's weights beside them
                 const float m12 = 12.0f - m;
                 uint32_t ph[NK][8], pl[NK][8];
                 at_f16v sn[NK];
-                {
+                float s0 = 0.0f, s1 = 0.0f;
+                auto weigh = [&](int n) { // score pair n's weights
+                    const int k = n >> 3, i = 2 * (n & 7);
+                    const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i], scale2, m12));
+                    const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i + 1], scale2, m12));
+                    s0 += e0;
+                    s1 += e1;
+                    const at_h2 p = __builtin_convertvector(at_f2{e0, e1}, at_h2);
+                    ph[k][i >> 1] = __builtin_bit_cast(uint32_t, p);
+                    pl[k][i >> 1] = __builtin_bit_cast(
+                        uint32_t, __builtin_convertvector(at_f2{at_less<0>(e0, p), at_less<1>(e1, p)}, at_h2));
+                };
+                if (KT * (t + 1) < whi) { // uniform over the wave
+                    // the next tile's scores on the matrix cores, this one's weights beside them
                     const unsigned char *kb = kv[(t + 1) & 1][0];
                     at_h8 kf[2][NK];
 #pragma unroll
                     for (int k = 0; k < NK; k++) {
                         kf[0][k] = *reinterpret_cast<const at_h8 *>(kb + ka[0] + 32 * k * RB);
                     }
-                    float s0 = 0.0f, s1 = 0.0f;
                     constexpr int PAIRS = NK * 8 / NJ < 1 ? 1 : NK * 8 / NJ; // score pairs a step
 #pragma unroll
                     for (int j = 0; j < NJ; j++) {
@@ -274,21 +286,27 @@ __device__ static inline void attn_tile_body(const AttnRowsArgs &a) {
                         for (int k = 0; k < NK; k++)
                             sn[k] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[j & 1][k], q[j], j ? sn[k] : at_f16v{}, 0, 0, 0);
 #pragma unroll
-                        for (int n = j * PAIRS; n < (j + 1) * PAIRS && n < 8 * NK; n++) {
-                            const int k = n >> 3, i = 2 * (n & 7);
-                            const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i], scale2, m12));
-                            const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i + 1], scale2, m12));
-                            s0 += e0;
-                            s1 += e1;
-                            const at_h2 p = __builtin_convertvector(at_f2{e0, e1}, at_h2);
-                            ph[k][i >> 1] = __builtin_bit_cast(uint32_t, p);
-                            pl[k][i >> 1] = __builtin_bit_cast(
-                                uint32_t, __builtin_convertvector(at_f2{at_less<0>(e0, p), at_less<1>(e1, p)}, at_h2));
-                        }
+                        for (int n = j * PAIRS; n < (j + 1) * PAIRS && n < 8 * NK; n++) weigh(n);
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    l += s0 + s1;
+                } else { // the wave's last tile: no next one; 16 keys past its ranges have weights of zero
+#pragma unroll
+                    for (int s = 0; s < KT / 16; s++) {
+                        if (s && KT * t + 16 * s >= whi) {
+#pragma unroll
+                            for (int n = 4 * s; n < 4 * s + 4; n++) ph[n >> 3][n & 7] = pl[n >> 3][n & 7] = 0;
+                            continue;
+                        }
+#pragma unroll
+                        for (int n = 4 * s; n < 4 * s + 4; n++) {
+                            weigh(n);
+                            if (n & 1) __builtin_amdgcn_sched_barrier(0); // (spills otherwise)
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < NK; k++) sn[k] = st[k];
                 }
+                l += s0 + s1;
                 const unsigned char *vb = kv[t & 1][1];
                 typedef __attribute__((address_space(3))) at_s4 *lds4;
                 auto value = [&](int d, int s) { // columns 32 d .. of keys 16 s .. 16 s + 15
