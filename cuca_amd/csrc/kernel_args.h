@@ -235,7 +235,7 @@ typedef struct {
 
 /* The quantized matmul on the matrix cores (qgemm.hip): out[t][n] =
  * x[t] . w[n] over f16 weights f16(d * q) and f16 activations, f32
- * accumulation; workgroups of 256 weight rows x 128 (MoE: or 64) tokens. */
+ * accumulation; workgroups of 256 weight rows x 128 or 64 tokens. */
 typedef struct {
     const uint8_t *w, *w_up;    /* packed weights (gate/up for GLU)          */
     const void *x;              /* [m][ldx] f32 or f16                       */

@@ -42,9 +42,12 @@
 // 1260 for the kernel before this one, 128 x 128 tiles of 32 x 32 x 16
 // products), down 468-483 (794), q/o 142-149 (219).  Q8_0: 990-1000, 543-550
 // and 165-167.  What bounds it: the products (two waves a SIMD take turns);
-// Q8_0's loads carry twice the bytes.  Not faster: tiles of 64 tokens in
-// place of a split k where the grid is small (down at 777 rows 136 -> 150
-// us); a second register set for the next chunk's weights spilled.
+// Q8_0's loads carry twice the bytes.  Not faster: a second register set for the
+// next chunk's weights spilled.  Tiles of 64 tokens (half the products a
+// dequantised weight) where tiles of 128 leave compute units idle and k is too
+// short to split, and past 64 rows where qgemm_few.hip's tiles take turns
+// (runtime.cpp, qgemm_common); where k splits they are slower (down at 777 rows
+// 136 -> 150 us).
 #include "common.h"
 #include <type_traits>
 
@@ -187,13 +190,22 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     // XCD x (workgroups x, x + 8, ...) takes row tiles x, x + 8, ... in
     // groups of 8; a group's workgroups take its row tiles in turn, token
     // tile by token tile, so that the workgroups resident on the XCD at once
-    // share their weight and activation tiles in its L2
+    // share their weight and activation tiles in its L2.  Fewer than eight
+    // row tiles would leave XCDs idle: there the tiles go round in turn (256 x
+    // 2048 at 777 rows 27.7 -> 23.5 us).
     const int id = blockIdx.x, xcd = id & 7, kq = id >> 3;
-    const int n_rx = (a.n_rt - xcd + 7) >> 3; // row tiles of this XCD
-    const int g = kq / (8 * a.n_ct), w = kq - g * 8 * a.n_ct;
-    const int gsz = min(8, n_rx - 8 * g);
-    if (gsz <= 0) return;
-    const int ct = w / gsz, rt = (8 * g + (w - ct * gsz)) * 8 + xcd;
+    int ct, rt;
+    if (a.n_rt < 8) {
+        ct = id / a.n_rt;
+        rt = id - ct * a.n_rt;
+    } else {
+        const int n_rx = (a.n_rt - xcd + 7) >> 3; // row tiles of this XCD
+        const int g = kq / (8 * a.n_ct), w = kq - g * 8 * a.n_ct;
+        const int gsz = min(8, n_rx - 8 * g);
+        if (gsz <= 0) return;
+        ct = w / gsz;
+        rt = (8 * g + (w - ct * gsz)) * 8 + xcd;
+    }
     if (ct >= a.n_ct) return;
     // routed experts: the tile's expert and pairs (uniform); tiles past the
     // last are empty
@@ -504,6 +516,17 @@ CUCA_QGEMM_TILE(cuca_qgemm_q4_0_split, float, 0, 8, false, 0, true)
 CUCA_QGEMM_TILE(cuca_qgemm_q8_0_split, float, 1, 8, false, 0, true)
 CUCA_QGEMM_TILE(cuca_qgemm_glu_q4_0_split, float, 0, 8, true, 0, true)
 CUCA_QGEMM_TILE(cuca_qgemm_glu_q8_0_split, float, 1, 8, true, 0, true)
+// tiles of 64 tokens
+#define CUCA_QGEMM_T64(TN, T, FN, FMT)                                                     \
+    CUCA_QGEMM_TILE(cuca_qgemm_##TN##_##FN##_t64, T, FMT, 4, false, 0, false)              \
+    CUCA_QGEMM_TILE(cuca_qgemm_glu_##TN##_##FN##_silu_t64, T, FMT, 4, true, 0, false)      \
+    CUCA_QGEMM_TILE(cuca_qgemm_glu_##TN##_##FN##_gelu_t64, T, FMT, 4, true, 1, false)
+CUCA_QGEMM_T64(f32, float, q4_0, 0)
+CUCA_QGEMM_T64(f32, float, q8_0, 1)
+CUCA_QGEMM_T64(f16, _Float16, q4_0, 0)
+CUCA_QGEMM_T64(f16, _Float16, q8_0, 1)
+CUCA_QGEMM_TILE(cuca_qgemm_q4_0_split_t64, float, 0, 4, false, 0, true)
+CUCA_QGEMM_TILE(cuca_qgemm_glu_q4_0_split_t64, float, 0, 4, true, 0, true)
 extern "C" __global__ __launch_bounds__(256) void cuca_qgemm_moe_plan(QGemmArgs a) { qgemm_moe_plan_body(a); }
 #define CUCA_QGEMM_MOE_TM(TN, T, FN, FMT, TM)                                              \
     CUCA_QGEMM_TILE(cuca_qgemm_moe_up_##TN##_##FN##_silu_t##TM, T, FMT, TM / 16, true, 0, false, 1) \

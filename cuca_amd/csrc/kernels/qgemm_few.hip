@@ -24,12 +24,14 @@
 //
 // Measured on MI355X, Q4_0, Llama-3-8B shapes, f32 rows, whole call, 32 / 64
 // / 128 rows against the tiled kernel that served them before: gate+up with
-// SwiGLU 27 / 40 / 72 us (53 / 74 / 121), down 21 / 30 / 39 (29 / 35 / 48),
-// q/o 14 / 20 / 24 (17 / 22 / 35), Q|K|V 15 / 22 / 30 (22 / 31 / 45).  What
-// bounds it: the dequantisation, about 14 vector instructions a block and
-// row tile (with every group's weights read from one cached address it runs
-// no faster), then, for the small weights, the two launches.  Two
-// groups of weights or activations in flight instead of one: no faster.
+// SwiGLU 24 / 37 us (47 / 69; at 128 rows qgemm.hip's tiles of 64 tokens take it),
+// down 19 / 28 / 37 (27 / 32 / 46), q/o 13 / 20 / 24 (16 / 23 / 34), Q|K|V 15 / 22 /
+// 29 (21 / 31 / 45).  What bounds it: one workgroup fits a compute unit (204
+// registers at 32 tokens), two waves a SIMD that meet at a barrier a packing
+// group, so loads, dequantisation (about 14 vector instructions a block and row
+// tile) and products take turns; then, for the small weights, the second launch
+// of the sums.  Two groups of weights or activations in flight instead of one: no
+// faster.
 //
 // Few weight tiles (grid y > 1): k is cut into ranges of whole groups and
 // each range's sums go to its own rows of the workspace, which
@@ -113,10 +115,13 @@ __device__ static inline void qgemm_few_body(const QGemmFewArgs &a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, u = lane >> 4;
     // workgroup id = 8 (n_ct (wt / 8) + token tile) + wt % 8: the token tiles
-    // of a weight tile run on one XCD and read its weights from HBM once
-    const int chunk = (int)blockIdx.x >> 3, wt = chunk / a.n_ct * 8 + ((int)blockIdx.x & 7);
-    if (wt >= a.n_tile) return; // the whole workgroup
-    const int t0 = chunk % a.n_ct * (NT * 16);
+    // of a weight tile run on one XCD and read its weights from HBM once.  Fewer
+    // than eight weight tiles would leave XCDs idle: there they go round in turn.
+    const int id = blockIdx.x, chunk = id >> 3;
+    const bool turn = a.n_tile < 8;
+    const int wt = turn ? id % a.n_tile : chunk / a.n_ct * 8 + (id & 7), ct = turn ? id / a.n_tile : chunk % a.n_ct;
+    if (wt >= a.n_tile || ct >= a.n_ct) return; // the whole workgroup
+    const int t0 = ct * (NT * 16);
     const int c0 = GLU ? wt * 64 + (wave & 3) * 16 : wt * 128 + wave * 16; // the wave's first output column
     const int row = min(c0 + r, a.rows - 1);
     const uint8_t *wr = (GLU && wave >= 4 ? a.w_up : a.w) + (int64_t)row * a.row_bytes;

@@ -2303,6 +2303,28 @@ cuca_status cuca_hip_qgemm_workspace(uint32_t ggml_type, int64_t n, int64_t k, i
 // (two where the rows are rounded to f16 first).
 constexpr int64_t kQgFewRows = 128;
 
+// Tokens a tile of the few-row kernels, and the workgroups that an XCD's
+// compute units have of their unsplit tiles at most (one runs on a compute
+// unit at once): a weight tile's workgroups stay on one XCD, so counted over the
+// chip 42 weight tiles were split into 252 workgroups for 256 units, 36 of them
+// on two XCDs of 32 (5376 x 21504 Q4_0 at 64 rows 62.5 us, in 5 splits 48).
+static int qgemm_few_tokens(int64_t m) { return m <= 16 ? 16 : m <= 32 ? 32 : 64; }
+static int64_t qgemm_few_load(int64_t rows, int64_t m, int glu) {
+    const int64_t wide = glu ? 64 : 128, tile = qgemm_few_tokens(m); // output columns a workgroup
+    const int64_t n_tile = (rows + wide - 1) / wide, n_ct = (m + tile - 1) / tile;
+    return n_tile < 8 ? (n_tile * n_ct + 7) / 8 : (n_tile + 7) / 8 * n_ct;
+}
+// From 65 rows on the tiled kernel where these take turns: a compute unit holds
+// two of its workgroups of 256 weight rows x 64 tokens.  Q4_0, 128 rows, us, few /
+// tiled: 32000 x 4096 73 / 61, gate and up 14336 x 4096 70 / 56, 5376 x 21504 (two
+// splits) 80 / 63; 6144 x 4096 (two splits of a short k) 29 / 30.  Q8_0, whose
+// weights are twice the bytes: 5376 x 21504 91 / 112.
+static bool qgemm_few_wins(const cuca_hip_ctx *ctx, bool q8, int64_t rows, int64_t k, int64_t m, int glu) {
+    if (m > kQgFewRows) return false;
+    const int64_t load = qgemm_few_load(rows, m, glu), units = ctx->cu_count / 8;
+    return m <= 64 || q8 || load <= (k >= 8192 ? units / 3 : units / 2);
+}
+
 static cuca_status qgemm_few(cuca_hip_ctx *ctx, const void *w, const void *w_up, bool q8, int64_t k, int64_t row_bytes,
                              int group, const void *x, int64_t ldx, int64_t m, int64_t rows, int glu, float clamp,
                              void *ws, float *part, size_t part_bytes, void *out, int64_t out_ld,
@@ -2344,13 +2366,12 @@ static cuca_status qgemm_few(cuca_hip_ctx *ctx, const void *w, const void *w_up,
     }
     a.out = out;
     a.out_ld = out_ld;
-    const int ni = m <= 16 ? 0 : m <= 32 ? 1 : 2; // 16, 32, 64 tokens a tile
-    a.n_ct = (int32_t)((m + (16 << ni) - 1) / (16 << ni));
+    const int tile = qgemm_few_tokens(m), ni = tile == 16 ? 0 : tile == 32 ? 1 : 2;
+    a.n_ct = (int32_t)((m + tile - 1) / tile);
     const int64_t wide = glu ? 64 : 128; // output columns a workgroup
     a.n_tile = (int32_t)((rows + wide - 1) / wide);
     // split k where the tiles leave compute units idle
-    const int64_t tiles = (int64_t)a.n_tile * a.n_ct;
-    int64_t splits = std::min<int64_t>(kQgMaxSplits, std::max<int64_t>(1, ctx->cu_count / tiles));
+    int64_t splits = std::min<int64_t>(kQgMaxSplits, std::max<int64_t>(1, ctx->cu_count / 8 / qgemm_few_load(rows, m, glu)));
     splits = std::min<int64_t>(splits, (int64_t)(part_bytes / ((size_t)(glu ? 2 : 1) * (size_t)m * (size_t)rows * 4)));
     splits = std::max<int64_t>(1, std::min<int64_t>(splits, a.ng));
     a.gs = (int32_t)((a.ng + splits - 1) / splits);
@@ -2415,25 +2436,34 @@ static cuca_status qgemm_common(cuca_hip_ctx *ctx, const void *w, const void *w_
     if (ws_bytes < xp_bytes)
         return fail(ctx, CUCA_INVALID_ARG, "qgemm: workspace of %zu bytes, %zu needed (cuca_hip_qgemm_workspace)",
                     ws_bytes, xp_bytes);
-    if (m <= kQgFewRows)
-        return qgemm_few(ctx, w, w_up, ggml_type == CUCA_GGML_Q8_0, k, (kp / 32 / g) * gb, g, x, ldx, m, rows, glu, clamp,
+    const bool q8 = ggml_type == CUCA_GGML_Q8_0;
+    if (qgemm_few_wins(ctx, q8, rows, k, m, glu))
+        return qgemm_few(ctx, w, w_up, q8, k, (kp / 32 / g) * gb, g, x, ldx, m, rows, glu, clamp,
                          ws, reinterpret_cast<float *>(static_cast<char *>(ws) + xp_bytes), ws_bytes - xp_bytes, out,
                          out_ld, dtype);
     const int64_t wide = glu ? 128 : 256; // output columns a workgroup
     const int64_t n_rt = (rows + wide - 1) / wide;
-    constexpr int tm = 128;
+    const int64_t nkc = kp / 128, cus = ctx->cu_count;
+    // Tiles of 64 tokens for up to 128 rows, and where tiles of 128 would leave
+    // compute units idle and k is too short for splits to fill them: up to 1024
+    // values, or 2048 where tiles of 64 occupy three quarters of the units
+    // unsplit (2048 x 768 Q8_0 at 512 rows 23 -> 18 us, 2048 x 2048 at 2048 rows 53 ->
+    // 44; 2048 x 2048 at 1024, 128 tiles: 35 -> 42, 4096 x 4096 at 777: 62 -> 72)
+    const int64_t work64 = n_rt * ((m + 63) / 64), work128 = n_rt * ((m + 127) / 128);
+    const bool t64 = m <= kQgFewRows || (work128 < cus && (k <= 1024 || (k <= 2048 && 4 * work64 >= 3 * cus)));
+    const int tm = t64 ? 64 : 128;
     const int64_t n_ct = (m + tm - 1) / tm;
     const int64_t tiles = (n_rt + 7) / 8 * 8 * n_ct;
-    const int64_t nkc = kp / 128;
     if (tiles > 0x7fffffffll) return fail(ctx, CUCA_UNSUPPORTED, "qgemm: grid too large");
     // split k for grids smaller than the CU count: up to two workgroups per
     // CU (what the CUs hold at once), at least 4 k-chunks per split, within
     // the workspace given
     int64_t splits = 1;
     const size_t split_row = (size_t)(glu ? 2 : 1) * (size_t)m * (size_t)rows * 4;
-    const int64_t work = n_rt * n_ct;
-    if (m <= 2048 && work < ctx->cu_count) {
-        splits = std::min<int64_t>(kQgMaxSplits, std::min<int64_t>(2 * ctx->cu_count / work, nkc / 4));
+    if (m <= kQgFewRows || (m <= 2048 && work128 < cus && !t64)) {
+        // (up to 128 rows by the XCD: a row tile's workgroups stay on one)
+        const int64_t room = m <= kQgFewRows ? 2 * (cus / 8) / ((n_rt + 7) / 8 * n_ct) : 2 * cus / work128;
+        splits = std::min<int64_t>(kQgMaxSplits, std::min<int64_t>(room, nkc / 4));
         splits = std::min<int64_t>(splits, (int64_t)((ws_bytes - xp_bytes) / split_row));
         if (splits < 2) splits = 1;
     }
@@ -2461,23 +2491,33 @@ static cuca_status qgemm_common(cuca_hip_ctx *ctx, const void *w, const void *w_
     a.clamp = clamp > 0.0f ? clamp : 0.0f;
     a.mp = (int32_t)(n_ct * tm);
     a.vec = out_ld % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & (dtype == CUCA_F16 ? 7u : 15u)) == 0;
-    const bool f16 = dtype == CUCA_F16, q8 = ggml_type == CUCA_GGML_Q8_0;
+    const bool f16 = dtype == CUCA_F16;
     static const Kernel prep_k[2][2] = {{cuca_qgemm_prep_f32_q4_0, cuca_qgemm_prep_f32_q8_0},
                                         {cuca_qgemm_prep_f16_q4_0, cuca_qgemm_prep_f16_q8_0}};
     if ((st = launch(ctx, prep_k[f16][q8], div_up((int64_t)a.mp * nkc * 16, CUCA_BLOCK_THREADS), CUCA_BLOCK_THREADS, 0,
                      a)) != CUCA_OK)
         return st;
-    // [dtype][format][plain, silu, gelu]
-    static const Kernel table_k[2][2][3] = {
-        {{cuca_qgemm_f32_q4_0, cuca_qgemm_glu_f32_q4_0_silu, cuca_qgemm_glu_f32_q4_0_gelu},
-         {cuca_qgemm_f32_q8_0, cuca_qgemm_glu_f32_q8_0_silu, cuca_qgemm_glu_f32_q8_0_gelu}},
-        {{cuca_qgemm_f16_q4_0, cuca_qgemm_glu_f16_q4_0_silu, cuca_qgemm_glu_f16_q4_0_gelu},
-         {cuca_qgemm_f16_q8_0, cuca_qgemm_glu_f16_q8_0_silu, cuca_qgemm_glu_f16_q8_0_gelu}}};
-    // [format][plain, glu]
+    // [dtype][format][plain, silu, gelu][128, 64 tokens a tile]
+    static const Kernel table_k[2][2][3][2] = {
+        {{{cuca_qgemm_f32_q4_0, cuca_qgemm_f32_q4_0_t64},
+          {cuca_qgemm_glu_f32_q4_0_silu, cuca_qgemm_glu_f32_q4_0_silu_t64},
+          {cuca_qgemm_glu_f32_q4_0_gelu, cuca_qgemm_glu_f32_q4_0_gelu_t64}},
+         {{cuca_qgemm_f32_q8_0, cuca_qgemm_f32_q8_0_t64},
+          {cuca_qgemm_glu_f32_q8_0_silu, cuca_qgemm_glu_f32_q8_0_silu_t64},
+          {cuca_qgemm_glu_f32_q8_0_gelu, cuca_qgemm_glu_f32_q8_0_gelu_t64}}},
+        {{{cuca_qgemm_f16_q4_0, cuca_qgemm_f16_q4_0_t64},
+          {cuca_qgemm_glu_f16_q4_0_silu, cuca_qgemm_glu_f16_q4_0_silu_t64},
+          {cuca_qgemm_glu_f16_q4_0_gelu, cuca_qgemm_glu_f16_q4_0_gelu_t64}},
+         {{cuca_qgemm_f16_q8_0, cuca_qgemm_f16_q8_0_t64},
+          {cuca_qgemm_glu_f16_q8_0_silu, cuca_qgemm_glu_f16_q8_0_silu_t64},
+          {cuca_qgemm_glu_f16_q8_0_gelu, cuca_qgemm_glu_f16_q8_0_gelu_t64}}}};
+    // [plain, glu]: tiles of 64 (Q4_0 alone); [format][plain, glu]: of 128
+    static const Kernel split64_k[2] = {cuca_qgemm_q4_0_split_t64, cuca_qgemm_glu_q4_0_split_t64};
     static const Kernel split_k[2][2] = {{cuca_qgemm_q4_0_split, cuca_qgemm_glu_q4_0_split},
                                          {cuca_qgemm_q8_0_split, cuca_qgemm_glu_q8_0_split}};
-    if (splits == 1) return launch(ctx, table_k[f16][q8][glu], (unsigned)tiles, 256, 0, a);
-    if ((st = launch2(ctx, split_k[q8][glu != 0], (unsigned)tiles, (unsigned)splits, 256, 0, a)) != CUCA_OK)
+    if (splits == 1) return launch(ctx, table_k[f16][q8][glu][t64], (unsigned)tiles, 256, 0, a);
+    if ((st = launch2(ctx, t64 ? split64_k[glu != 0] : split_k[q8][glu != 0], (unsigned)tiles, (unsigned)splits, 256, 0,
+                      a)) != CUCA_OK)
         return st;
     static const Kernel red_k[2][3] = {{cuca_qgemm_reduce_f32, cuca_qgemm_reduce_glu_f32_silu, cuca_qgemm_reduce_glu_f32_gelu},
                                        {cuca_qgemm_reduce_f16, cuca_qgemm_reduce_glu_f16_silu, cuca_qgemm_reduce_glu_f16_gelu}};

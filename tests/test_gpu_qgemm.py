@@ -180,3 +180,59 @@ def test_qgemm_over_its_own_activations(ctx, dtype, m):
     want = xf @ w.T
     tol = bound(xf, w, k) + (2.0 ** -11 * np.abs(want) if dtype == "f16" else 0.0)
     assert np.all(np.abs(buf.numpy().astype(np.float64) - want) <= tol)
+
+
+def launched(ctx, call):
+    ctx.profile_start(8)
+    call()
+    return [name for name, _ in ctx.profile_stop()]
+
+
+@pytest.mark.parametrize("qtype,n,k,m,kernels", [
+    # past 64 rows where the few-row kernels would take turns: split and unsplit
+    ("q4_0", 8330, 2080, 65, ("prep_f32_q4_0", "q4_0_split_t64", "reduce_f32")),
+    ("q4_0", 8330, 96, 128, ("prep_f32_q4_0", "f32_q4_0_t64")),
+    ("q4_0", 5250, 8192, 70, ("prep_f32_q4_0", "q4_0_split_t64", "reduce_f32")),
+    ("q4_0", 8190, 96, 65, ("rows_f32", "few_f16_f32_q4_0_n4")),
+    ("q8_0", 8330, 96, 65, ("rows_f32", "few_f16_f32_q8_0_n4")),
+    # few tiles of 128 of a k too short to split
+    ("q8_0", 2040, 768, 161, ("prep_f32_q8_0", "f32_q8_0_t64")),
+    ("q8_0", 2040, 1056, 161, ("prep_f32_q8_0", "q8_0_split", "reduce_f32")),
+    ("q4_0", 2040, 2048, 1537, ("prep_f32_q4_0", "f32_q4_0_t64"))])
+def test_qgemm_tiles_of_64_tokens(ctx, qtype, n, k, m, kernels):
+    raw, wt, x = setup(ctx, qtype, n, k, m, "f32", n + k + m)
+    dx, out = ctx.array(x), ctx.empty((m, n), np.float32)
+    wsb = hip.qgemm_workspace(QT[qtype], n, k, m)
+    ws = ctx.empty((wsb,), np.uint8)
+    names = launched(ctx, lambda: ctx.qgemm(wt.packed.ptr, QT[qtype], n, k, dx.ptr, k, m, n, ws.ptr, wsb, out.ptr, n,
+                                            hip.F32))
+    assert names == ["cuca_qgemm_" + s for s in kernels]
+    w, xf = dense(raw, qtype, n, k), x.astype(np.float64)
+    assert np.all(np.abs(out.numpy() - xf @ w.T) <= bound(xf, w, k) + 1e-30)
+
+
+@pytest.mark.parametrize("act", [hip.ACT_SILU, hip.ACT_GELU_TANH])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("qtype,n,k,m", [("q4_0", 200, 480, 129), ("q8_0", 131, 96, 200), ("q4_0", 4170, 1056, 66),
+                                         ("q4_0", 4170, 64, 100)])
+def test_qgemm_glu_tiles_of_64_tokens(ctx, qtype, dtype, act, n, k, m):
+    rng = np.random.default_rng(n + k + m)
+    graw, uraw = (W.quant_table(rng, n, k, qtype, (0.004, 0.03)) for _ in range(2))
+    gw, uw = (ops.QmmWeight.from_raw(ctx, QT[qtype], r, n, k) for r in (graw, uraw))
+    x = (rng.standard_normal((m, k)) * 0.5).astype(NP[dtype])
+    dx, out = ctx.array(x), ctx.empty((m, n), NP[dtype])
+    wsb = hip.qgemm_workspace(QT[qtype], n, k, m, glu=True)
+    ws = ctx.empty((wsb,), np.uint8)
+    names = launched(ctx, lambda: ctx.qgemm_glu(gw.packed.ptr, uw.packed.ptr, QT[qtype], n, k, dx.ptr, k, m, act, 0.0,
+                                                ws.ptr, wsb, out.ptr, n, hip.dtype_code(NP[dtype])))
+    assert names[1].endswith("_t64"), names
+    xf, wg, wu = x.astype(np.float64), dense(graw, qtype, n, k), dense(uraw, qtype, n, k)
+    g, u, bg, bu = xf @ wg.T, xf @ wu.T, bound(xf, wg, k), bound(xf, wu, k)
+    if act == hip.ACT_SILU:
+        a = g / (1.0 + np.exp(-g))
+    else:
+        a = 0.5 * g * (1.0 + np.tanh(np.sqrt(2.0 / np.pi) * (g + 0.044715 * g ** 3)))
+    want = a * u
+    tol = 1.2 * bg * (np.abs(u) + bu) + np.abs(a) * bu + (1e-5 if dtype == "f32" else 2.0 ** -10) * np.abs(want) + 1e-30
+    err = np.abs(out.numpy().astype(np.float64) - want)
+    assert np.all(err <= tol), float(np.max(err / tol))
