@@ -19,6 +19,8 @@
 // LDS busy with the reads all the time.  Two workgroups fit a compute unit,
 // two waves a SIMD, so that one wave's dequantisation (about 14 vector
 // instructions an operand of 8 products) runs under the other's products.
+// Down of the routed experts, whose grids are smaller, also takes 128 weight rows
+// a workgroup, 32 a wave (RI = 2; runtime.cpp, moe_qgemm_common).
 //
 // k order.  The weights are read in the packed layout of qmm.hip.  A dot
 // product may sum its terms in any order, so the k index of the operands is
@@ -56,7 +58,6 @@ typedef _Float16 qg_h8 __attribute__((ext_vector_type(8)));
 typedef float qg_acc __attribute__((ext_vector_type(4)));
 typedef uint32_t qg_u2 __attribute__((ext_vector_type(2)));
 
-#define QG_ROWS 256       // weight rows per workgroup (64 per wave)
 #define QG_KC 128         // values per k-chunk: 4 k-steps of 32
 
 template <int FMT> struct QgFmt;
@@ -177,11 +178,12 @@ template <typename T, int FMT> __device__ static inline void qgemm_prep_body(con
 // writes its f32 sums to the partial rows of the workspace (qgemm_reduce
 // adds the splits in order and applies the epilogue); otherwise the
 // epilogue is applied here.
-template <typename T, int FMT, int NT, bool GLU, int ACT, bool SPLIT, int MOE = 0>
+template <typename T, int FMT, int NT, bool GLU, int ACT, bool SPLIT, int MOE = 0, int RI = 4>
 __device__ static inline void qgemm_body(const QGemmArgs &a) {
     using F = QgFmt<FMT>;
     constexpr int TM = NT * 16;
-    constexpr int COLS = GLU ? QG_ROWS / 2 : QG_ROWS; // output columns of a workgroup
+    static_assert(!GLU || RI == 4, "gate, gate, up, up");
+    constexpr int COLS = 64 * RI / (GLU ? 2 : 1); // output columns of a workgroup
     // two buffers of a k-chunk's activations: rows of 256 bytes, 16-byte unit
     // v of row R at unit v ^ (R & 7), so that the reads of 8 rows at one unit
     // fall in different banks
@@ -225,9 +227,9 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     const int tok0 = ct * TM;
     const int n0 = rt * COLS + wave * (COLS / 4); // the wave's first output column
     // the wave's 16-row tiles (GLU: gate, gate, up, up of the same columns)
-    QgTile tile[4];
+    QgTile tile[RI];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < RI; i++) {
         const int r0 = n0 + 16 * (GLU ? i & 1 : i); // uniform
         const int left = max(0, min(16, a.rows - r0));
         const uint64_t p = (uint64_t)(uintptr_t)(GLU && i >= 2 ? a.w_up : a.w) + (uint64_t)((int64_t)r0 * a.row_bytes) +
@@ -258,15 +260,15 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
             lds_copy16(off[i & 1], src, dst);
         }
     };
-    qg_acc acc[4][NT];
+    qg_acc acc[RI][NT];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RI; i++)
 #pragma unroll
         for (int j = 0; j < NT; j++) acc[i][j] = qg_acc{};
     // weights: a tile's next chunk is requested into its own registers, right
     // after the last operand made from them (a second register set, a chunk
     // ahead, spilled)
-    QgW<FMT> wv[4];
+    QgW<FMT> wv[RI];
     auto load = [&](int kc, int i, int unit) {
         const int c = kc < kc1 ? kc : kc1 - 1; // (the last again past the end, unused)
         wv[i].c[unit] = qg_load<FMT>(tile[i], c, unit, woff);
@@ -281,7 +283,7 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     };
     constexpr int STEPS = 4 / F::UNITS; // k-steps a load
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < RI; i++)
 #pragma unroll
         for (int q = 0; q < F::UNITS; q++) load(kc0, i, q);
     copy(kc0, 0);
@@ -297,10 +299,10 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
         for (int s = 0; s < 4; s++) {
             if (s % STEPS == 0) {
 #pragma unroll
-                for (int i = 0; i < 4; i++) qg_transpose(wv[i].c[s / STEPS]);
+                for (int i = 0; i < RI; i++) qg_transpose(wv[i].c[s / STEPS]);
             }
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < RI; i++) {
                 const qg_h8 av = qg_dequant<FMT>(wv[i], s);
                 if (s % STEPS == STEPS - 1) {
                     __builtin_amdgcn_sched_barrier(0);
@@ -309,7 +311,7 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
 #pragma unroll
                 for (int j = 0; j < NT; j++) {
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, b[j], acc[i][j], 0, 0, 0);
-                    if (i == 3 && s < 3) read(buf, s + 1, j); // the next k-step's operand
+                    if (i == RI - 1 && s < 3) read(buf, s + 1, j); // the next k-step's operand
                 }
                 // an operand is dequantised no further ahead (the kernels spill otherwise)
                 __builtin_amdgcn_sched_barrier(0);
@@ -319,15 +321,14 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
         // this buffer.  Of a wave's loads only the weight loads above come
         // after its copies (a load does not pass an asm with a memory
         // clobber), so that many may stay in flight.
-        if constexpr (F::UNITS == 1) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((F::UNITS + 1) * RI) : "memory");
         __syncthreads();
     }
     // accumulator e of lane (r, u) in tile (i, j): weight row 16 i + 4 u + e
     // of the wave's, token 16 j + r.  The empty asm keeps a tile where it is
     // until its turn (copied out all at once, the tiles would set the
     // kernel's register count).
-    constexpr int NI = GLU && !SPLIT ? 2 : 4;
+    constexpr int NI = GLU && !SPLIT ? 2 : RI;
 #pragma unroll
     for (int j = 0; j < NT; j++) {
         const int local = 16 * j + r;
@@ -336,7 +337,7 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
             asm volatile("" : "+v"(acc[i][j]));
-            if (GLU && !SPLIT) asm volatile("" : "+v"(acc[i + 2][j]));
+            if constexpr (GLU && !SPLIT) asm volatile("" : "+v"(acc[i + 2][j]));
             if (!live) continue;
             const int c = n0 + 16 * (GLU ? i & 1 : i) + 4 * u;
             if (SPLIT) { // partial rows: [split][gate, up][m][rows] f32
@@ -355,7 +356,7 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 v[e] = acc[i][j][e];
-                if (GLU) {
+                if constexpr (GLU) {
                     float gg = v[e], uu = acc[(i + 2) & 3][j][e];
                     if (a.clamp > 0.0f) { // Glu::apply's clamp (cpu.rs:364-368)
                         gg = fminf(gg, a.clamp);
@@ -528,14 +529,20 @@ CUCA_QGEMM_T64(f16, _Float16, q8_0, 1)
 CUCA_QGEMM_TILE(cuca_qgemm_q4_0_split_t64, float, 0, 4, false, 0, true)
 CUCA_QGEMM_TILE(cuca_qgemm_glu_q4_0_split_t64, float, 0, 4, true, 0, true)
 extern "C" __global__ __launch_bounds__(256) void cuca_qgemm_moe_plan(QGemmArgs a) { qgemm_moe_plan_body(a); }
-#define CUCA_QGEMM_MOE_TM(TN, T, FN, FMT, TM)                                              \
+#define CUCA_QGEMM_MOE_UP(TN, T, FN, FMT, TM)                                              \
     CUCA_QGEMM_TILE(cuca_qgemm_moe_up_##TN##_##FN##_silu_t##TM, T, FMT, TM / 16, true, 0, false, 1) \
-    CUCA_QGEMM_TILE(cuca_qgemm_moe_up_##TN##_##FN##_gelu_t##TM, T, FMT, TM / 16, true, 1, false, 1) \
-    CUCA_QGEMM_TILE(cuca_qgemm_moe_down_##TN##_##FN##_t##TM, T, FMT, TM / 16, false, 0, false, 2)
+    CUCA_QGEMM_TILE(cuca_qgemm_moe_up_##TN##_##FN##_gelu_t##TM, T, FMT, TM / 16, true, 1, false, 1)
+#define CUCA_QGEMM_MOE_DOWN(TN, T, FN, FMT, TM)                                            \
+    CUCA_QGEMM_TILE(cuca_qgemm_moe_down_##TN##_##FN##_r128_t##TM, T, FMT, TM / 16, false, 0, false, 2, 2)
 #define CUCA_QGEMM_MOE_SET(TN, T, FN, FMT)                                                 \
     CUCA_QGEMM(cuca_qgemm_moe_prep_##TN##_##FN, qgemm_moe_prep_body, T, FMT)               \
-    CUCA_QGEMM_MOE_TM(TN, T, FN, FMT, 64)                                                  \
-    CUCA_QGEMM_MOE_TM(TN, T, FN, FMT, 128)
+    CUCA_QGEMM_MOE_UP(TN, T, FN, FMT, 32)                                                  \
+    CUCA_QGEMM_MOE_UP(TN, T, FN, FMT, 64)                                                  \
+    CUCA_QGEMM_MOE_UP(TN, T, FN, FMT, 128)                                                 \
+    CUCA_QGEMM_MOE_DOWN(TN, T, FN, FMT, 32)                                                \
+    CUCA_QGEMM_MOE_DOWN(TN, T, FN, FMT, 64)                                                \
+    CUCA_QGEMM_MOE_DOWN(TN, T, FN, FMT, 128)                                               \
+    CUCA_QGEMM_TILE(cuca_qgemm_moe_down_##TN##_##FN##_t128, T, FMT, 8, false, 0, false, 2)
 CUCA_QGEMM_MOE_SET(f32, float, q4_0, 0)
 CUCA_QGEMM_MOE_SET(f32, float, q8_0, 1)
 CUCA_QGEMM_MOE_SET(f16, _Float16, q4_0, 0)

@@ -2932,11 +2932,24 @@ static cuca_status moe_qgemm_common(cuca_hip_ctx *ctx, const void *w, const void
     if (ws_bytes < need)
         return fail(ctx, CUCA_INVALID_ARG, "moe qgemm: workspace of %zu bytes, %zu needed (cuca_hip_moe_qgemm_workspace)",
                     ws_bytes, need);
-    const int tm = moe_qgemm_tm(max_pairs, n_experts);
+    // Pairs a tile and weight rows a workgroup.  The workspace is that of
+    // moe_qgemm_tm's tiles; smaller ones, for experts of few pairs, fit in it.
+    // Down of tiles under 128 pairs, and of a grid that leaves compute units idle
+    // or XCDs uneven: workgroups of 128 rows.  MI355X, us, by 128 rows and 32, 64
+    // pairs / by 256 rows and 64: 128 experts, 2048 x 768 Q4_0, 16 pairs an expert
+    // 86, 94 / 107, 64 pairs 134, 136 / 152 (Q8_0 158, 143 / 154); by 128 rows / 256,
+    // tiles of 128: 8 experts, 2048 x 8192, 256 pairs each 134 / 188, 512 316 / 294,
+    // 32 experts, 2880 x 2880, 128 each 193 / 213.  Up by tiles of 32 / 64 (128
+    // experts of 768 over 2048): 16 pairs 148 / 174, 24 171 / 179 (Q8_0 235 / 225).
+    const double mean = (double)max_pairs / (double)n_experts;
+    int tm = moe_qgemm_tm(max_pairs, n_experts);
+    if (tm == 64 && mean <= (up ? 16.0 : 32.0)) tm = 32;
     const int64_t tiles = moe_qgemm_tiles(max_pairs, n_experts, tm);
     const int64_t kp = qgemm_kp(g, k), nkc = kp / 128;
-    const int64_t wide = up ? 128 : 256; // output columns a workgroup
-    const int64_t n_rt = (n + wide - 1) / wide;
+    const int64_t n_256 = (n + 255) / 256, n_128 = (n + 127) / 128;
+    const bool uneven = n_256 >= 8 && (n_256 + 7) / 8 * 256 * 5 >= (n_128 + 7) / 8 * 128 * 6; // a fifth more on the fullest XCD
+    const bool r128 = !up && (tm < 128 || n_256 * tiles < ctx->cu_count || uneven);
+    const int64_t n_rt = up || r128 ? n_128 : n_256; // output columns a workgroup: 128 (gate and up) or 256
     const int64_t grid = (n_rt + 7) / 8 * 8 * tiles;
     if (grid > 0x7fffffffll || tiles * tm * nkc * 16 / CUCA_BLOCK_THREADS + 1 > 0x7fffffffll)
         return fail(ctx, CUCA_UNSUPPORTED, "moe qgemm: grid too large");
@@ -2981,21 +2994,25 @@ static cuca_status moe_qgemm_common(cuca_hip_ctx *ctx, const void *w, const void
     if ((st = launch(ctx, prep_k[f16][q8], div_up((int64_t)a.mp * nkc * 16, CUCA_BLOCK_THREADS), CUCA_BLOCK_THREADS,
                      0, a)) != CUCA_OK)
         return st;
-    // [dtype][format][down, up silu, up gelu][tile pairs 64, 128]
-    static const Kernel table_k[2][2][3][2] = {
-        {{{cuca_qgemm_moe_down_f32_q4_0_t64, cuca_qgemm_moe_down_f32_q4_0_t128},
-          {cuca_qgemm_moe_up_f32_q4_0_silu_t64, cuca_qgemm_moe_up_f32_q4_0_silu_t128},
-          {cuca_qgemm_moe_up_f32_q4_0_gelu_t64, cuca_qgemm_moe_up_f32_q4_0_gelu_t128}},
-         {{cuca_qgemm_moe_down_f32_q8_0_t64, cuca_qgemm_moe_down_f32_q8_0_t128},
-          {cuca_qgemm_moe_up_f32_q8_0_silu_t64, cuca_qgemm_moe_up_f32_q8_0_silu_t128},
-          {cuca_qgemm_moe_up_f32_q8_0_gelu_t64, cuca_qgemm_moe_up_f32_q8_0_gelu_t128}}},
-        {{{cuca_qgemm_moe_down_f16_q4_0_t64, cuca_qgemm_moe_down_f16_q4_0_t128},
-          {cuca_qgemm_moe_up_f16_q4_0_silu_t64, cuca_qgemm_moe_up_f16_q4_0_silu_t128},
-          {cuca_qgemm_moe_up_f16_q4_0_gelu_t64, cuca_qgemm_moe_up_f16_q4_0_gelu_t128}},
-         {{cuca_qgemm_moe_down_f16_q8_0_t64, cuca_qgemm_moe_down_f16_q8_0_t128},
-          {cuca_qgemm_moe_up_f16_q8_0_silu_t64, cuca_qgemm_moe_up_f16_q8_0_silu_t128},
-          {cuca_qgemm_moe_up_f16_q8_0_gelu_t64, cuca_qgemm_moe_up_f16_q8_0_gelu_t128}}}};
-    return launch(ctx, table_k[f16][q8][up][tm == 128], (unsigned)grid, CUCA_BLOCK_THREADS, 0, a);
+    // [dtype][format][down of 128 rows, up silu, up gelu][tile pairs 32, 64, 128]
+    static const Kernel table_k[2][2][3][3] = {
+        {{{cuca_qgemm_moe_down_f32_q4_0_r128_t32, cuca_qgemm_moe_down_f32_q4_0_r128_t64, cuca_qgemm_moe_down_f32_q4_0_r128_t128},
+          {cuca_qgemm_moe_up_f32_q4_0_silu_t32, cuca_qgemm_moe_up_f32_q4_0_silu_t64, cuca_qgemm_moe_up_f32_q4_0_silu_t128},
+          {cuca_qgemm_moe_up_f32_q4_0_gelu_t32, cuca_qgemm_moe_up_f32_q4_0_gelu_t64, cuca_qgemm_moe_up_f32_q4_0_gelu_t128}},
+         {{cuca_qgemm_moe_down_f32_q8_0_r128_t32, cuca_qgemm_moe_down_f32_q8_0_r128_t64, cuca_qgemm_moe_down_f32_q8_0_r128_t128},
+          {cuca_qgemm_moe_up_f32_q8_0_silu_t32, cuca_qgemm_moe_up_f32_q8_0_silu_t64, cuca_qgemm_moe_up_f32_q8_0_silu_t128},
+          {cuca_qgemm_moe_up_f32_q8_0_gelu_t32, cuca_qgemm_moe_up_f32_q8_0_gelu_t64, cuca_qgemm_moe_up_f32_q8_0_gelu_t128}}},
+        {{{cuca_qgemm_moe_down_f16_q4_0_r128_t32, cuca_qgemm_moe_down_f16_q4_0_r128_t64, cuca_qgemm_moe_down_f16_q4_0_r128_t128},
+          {cuca_qgemm_moe_up_f16_q4_0_silu_t32, cuca_qgemm_moe_up_f16_q4_0_silu_t64, cuca_qgemm_moe_up_f16_q4_0_silu_t128},
+          {cuca_qgemm_moe_up_f16_q4_0_gelu_t32, cuca_qgemm_moe_up_f16_q4_0_gelu_t64, cuca_qgemm_moe_up_f16_q4_0_gelu_t128}},
+         {{cuca_qgemm_moe_down_f16_q8_0_r128_t32, cuca_qgemm_moe_down_f16_q8_0_r128_t64, cuca_qgemm_moe_down_f16_q8_0_r128_t128},
+          {cuca_qgemm_moe_up_f16_q8_0_silu_t32, cuca_qgemm_moe_up_f16_q8_0_silu_t64, cuca_qgemm_moe_up_f16_q8_0_silu_t128},
+          {cuca_qgemm_moe_up_f16_q8_0_gelu_t32, cuca_qgemm_moe_up_f16_q8_0_gelu_t64, cuca_qgemm_moe_up_f16_q8_0_gelu_t128}}}};
+    // [dtype][format]: down of 256 rows, tiles of 128 pairs
+    static const Kernel down_k[2][2] = {{cuca_qgemm_moe_down_f32_q4_0_t128, cuca_qgemm_moe_down_f32_q8_0_t128},
+                                        {cuca_qgemm_moe_down_f16_q4_0_t128, cuca_qgemm_moe_down_f16_q8_0_t128}};
+    const Kernel kern = up || r128 ? table_k[f16][q8][up][tm == 128 ? 2 : tm == 64] : down_k[f16][q8];
+    return launch(ctx, kern, (unsigned)grid, CUCA_BLOCK_THREADS, 0, a);
 }
 
 cuca_status cuca_hip_moe_up_qgemm(cuca_hip_ctx *ctx, const void *gate, const void *up, int64_t expert_stride,

@@ -67,6 +67,21 @@ def test_a_wait_state_stands_between_a_write_of_m0_and_the_lds_copy_that_reads_i
     assert copies > 0 and not bad, (copies, bad[:4])
 
 
+def test_the_routed_experts_small_tiles_fit_the_workspace_of_the_larger():
+    """The grouped matmul's workspace holds a plan of three words a tile and
+    its tiles' f16 rows, for tiles of 64 pairs (128 from 96 pairs an expert
+    on); calls of few pairs an expert run tiles of 32."""
+    for qt, group in ((hip.GGML_Q4_0, 512), (hip.GGML_Q8_0, 256)):
+        for k in (32, 256, 768, 2048):
+            for experts in (1, 2, 3, 8, 60, 128, 4096):
+                for pairs in sorted({1, 2, 31, 32, 33, 63, 64, 65, experts, 7 * experts + 1, 32 * experts}):
+                    if pairs > 32 * experts:
+                        continue
+                    tiles = -(-pairs // 32) + min(experts, pairs)
+                    need = -(-tiles * 12 // 256) * 256 + tiles * 32 * (-(-k // group) * group) * 2
+                    assert need <= hip.moe_qgemm_workspace(qt, k, experts, pairs), (k, experts, pairs)
+
+
 @pytest.mark.parametrize("spec", [
     dict(n_dims=128, base=1e6, positions=64),
     dict(n_dims=128, base=5e5, positions=8192),

@@ -202,3 +202,43 @@ def test_offsets_are_clamped_and_host_checks(ctx):
     with pytest.raises(hip.CucaError, match="experts"):
         ctx.moe_up_qgemm(eb.gate.ptr, eb.up.ptr, eb.stride_gu, hip.GGML_Q4_0, ff, n_embd, 5000, dx.ptr, n_embd, t,
                          bad_off.ptr, tok.ptr, 4, hip.ACT_SILU, 0.0, ws.ptr, wsb, hidden.ptr, ff, hip.F32)
+
+
+@pytest.mark.parametrize("qtype,dtype,act", [("q4_0", "f32", hip.ACT_SILU), ("q8_0", "f16", hip.ACT_GELU_TANH)])
+@pytest.mark.parametrize("counts,n,k,up,down", [
+    ([1, 0, 33, 5, 16, 31], 130, 96, "t32", "r128_t32"),     # 14 pairs an expert: full, partial and single tiles
+    ([40, 20, 1], 257, 544, "t64", "r128_t32"),              # 20
+    ([70, 33], 127, 288, "t64", "r128_t64"),                 # 51
+    ([130, 97], 300, 96, "t128", "r128_t128"),               # 113: a grid that leaves compute units idle
+    ([130, 97], 16385, 64, "t128", "t128"),                  # and one that does not
+    ([1800, 1799], 2049, 64, "t128", "r128_t128")])          # nine row tiles of 256: two on one XCD
+def test_moe_qgemm_tiles(ctx, qtype, dtype, act, counts, n, k, up, down):
+    rng = np.random.default_rng(n + k + len(counts))
+    npd = np.float16 if dtype == "f16" else np.float32
+    E, pairs = len(counts), sum(counts)
+    one = (hip.qweight_bytes(QT[qtype], n, k) + 15) // 16 * 16
+    raws = [[W.quant_table(rng, n, k, qtype, (0.004, 0.03)) for _ in range(3)] for _ in range(E)]
+    pools = [ctx.empty((E * one,), np.uint8) for _ in range(3)]
+    for e in range(E):
+        for pool, raw in zip(pools, raws[e]):
+            d = ctx.array(raw)
+            ctx.qweight_pack(d.ptr, QT[qtype], n, k, pool.ptr + e * one)
+            ctx.sync()
+    x = (0.3 * rng.standard_normal((pairs, k))).astype(npd)
+    tok, wt = rng.permutation(pairs).astype(np.int32), rng.uniform(0.05, 1.0, pairs).astype(np.float32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    dx, d_off, d_tok, d_wt = (ctx.array(v) for v in (x, offsets, tok, wt))
+    wsb = hip.moe_qgemm_workspace(QT[qtype], k, E, pairs)
+    ws = ctx.empty((wsb,), np.uint8)
+    hidden, scr = ctx.empty((pairs, n), npd), ctx.empty((pairs, n), np.float32)
+    ctx.profile_start(8)
+    ctx.moe_up_qgemm(pools[0].ptr, pools[1].ptr, one, QT[qtype], n, k, E, dx.ptr, k, pairs, d_off.ptr, d_tok.ptr, pairs,
+                     act, 0.0, ws.ptr, wsb, hidden.ptr, n, hip.dtype_code(npd))
+    ctx.moe_down_qgemm(pools[2].ptr, one, QT[qtype], n, k, E, dx.ptr, k, d_off.ptr, d_wt.ptr, pairs, ws.ptr, wsb,
+                       scr.ptr, n, hip.dtype_code(npd))
+    names = [name for name, _ in ctx.profile_stop()]
+    assert names[2].endswith(f"{'silu' if act == hip.ACT_SILU else 'gelu'}_{up}") and \
+        names[5] == f"cuca_qgemm_moe_down_{dtype}_{qtype}_{down}", names
+    sample = set(rng.choice(pairs, min(pairs, 200), replace=False).tolist())
+    check_up(hidden.numpy(), x, raws, qtype, offsets, tok, act, k, n, dtype, sample)
+    check_down(scr.numpy(), x, raws, qtype, offsets, wt, n, k, sample)
