@@ -27,13 +27,16 @@ Algorithmic bytes per unit (s = bytes per activation, H 4096, F 14336):
   glu         3 s F                    per row   (gate, up in; out)
 Per-call constants (gamma, norm weights) are counted once.
 
-`configs` repeats the step for the other workload configs (A Qwen3-0.6B,
+stdout is one short JSON line; everything else that was measured is one JSON
+object on stderr ("[bench] details: "), or in the file that --details names.
+
+There, `configs` repeats the step for the other workload configs (A Qwen3-0.6B,
 B Llama-3-8B decode batch, D Gemma-2-9B with the sandwich norms, GeGLU and
 interleaved RoPE, E Qwen3-30B-A3B with QK-norm RoPE and the ragged
 expert-grouped SwiGLU), each op's kernel GB/s from its timestamps.
-`prefill_bar` (near the end of the line) gathers every op's fraction of
-the HBM peak at the sizes of the 70 % bar (config C at 4096 and 16384
-tokens, config E at 8192), `decode_bar` the batch-1 decode figures.
+`prefill_bar` gathers every op's fraction of the HBM peak at the sizes of the
+70 % bar (config C at 4096 and 16384 tokens, config E at 8192).  `decode_bar`,
+on the line, has the batch-1 decode figures.
 
 roofline: the dominant kernel (SwiGLU) -- its algorithmic bytes per launch
 divided by its average launch duration over the timed steps, from the start
@@ -1577,6 +1580,8 @@ def main():
     ap.add_argument("--no-attn", action="store_true", help="skip the paged decode attention")
     ap.add_argument("--no-qmm", action="store_true",
                     help="skip the quantized matmuls, routed experts and LM head")
+    ap.add_argument("--details", metavar="FILE",
+                    help="write everything measured there as JSON (default: one line on stderr)")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU: these ops run on one GPU's share of the work and "
@@ -1772,6 +1777,15 @@ def main():
         "hbm_frac": round(value / HBM_PEAK_GBS, 4),
         "copy_gbs": round(copy_gbs, 1),
         "verified_rows": checked_rows,
+        "op_frac": {k: v["frac"] for k, v in ops.items()},
+        "decode_bar": decode_bar(decode, attn),
+        "roofline": {"kernel": glu["kernel"], "bound": "hbm", "achieved": glu["gbs"], "peak": HBM_PEAK_GBS,
+                     "unit": "GB/s", "frac": glu["frac"], "avg_launch_us": glu["us"]},
+        "cpu_baseline": cpu and {k: cpu[k] for k in ("value", "unit", "cores", "kind")},
+    }
+    # the line stays short; everything else that was measured goes to stderr, or
+    # to the file asked for
+    details = {
         "parity_raw": parity_raw,
         "ops": ops,
         f"prefill_{other}": big,
@@ -1787,14 +1801,15 @@ def main():
         "prefill_layer": player,
         "prefill_layer_dense": player_dense,
         "prefill_bar": prefill_bar(ops, args.tokens, big, configs),
-        "decode_bar": decode_bar(decode, attn),
-        "roofline": {"kernel": glu["kernel"], "bound": "hbm",
-                     "achieved": glu["gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": glu["frac"], "traffic": traffic,
-                     "traffic_source": traffic_src,
-                     "algorithmic_bytes_per_launch": glu["bytes"], "avg_launch_us": glu["us"]},
+        "roofline": {"traffic": traffic, "traffic_source": traffic_src,
+                     "algorithmic_bytes_per_launch": glu["bytes"]},
         "cpu_baseline": cpu,
     }
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(details, f, indent=1)
+    else:
+        log("details: " + json.dumps(details))
     print(json.dumps(out), flush=True)
     ctx.close()
 
