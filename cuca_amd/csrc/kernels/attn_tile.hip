@@ -32,15 +32,17 @@
 //    conversions, two matrix instructions and eight scores' arithmetic a step; a
 //    wave's last tile has none, and weighs only the 16 keys its ranges reach.
 //
-// What bounds it: the matrix cores are busy 57 % and the vector unit 48 % of
-// the time a compute unit works, at two waves a SIMD and about 1.9 GHz; each
-// wave alternates between them (a value product has no arithmetic to hide
-// behind) and waits at the tile's barrier a fifth of the time.  MI355X, us,
+// What bounds it (causal 4096 rows, 32 heads over 8 of 128): the matrix cores are
+// busy 44 % of the launch (SQ_VALU_MFMA_BUSY_CYCLES); each wave, two a SIMD,
+// alternates between them and the vector unit (a value product has no arithmetic
+// to hide behind), and waits for copies and the tile's barrier 23 % and for issue
+// 33 % of its time (SQ_WAIT_ANY, SQ_WAIT_INST_ANY / SQ_WAVE_CYCLES).  MI355X, us,
 // before (16-key blocks, 16x16x16 products, a row tile of 16) -> after: causal
-// 4096 rows of 32 heads over 8 of 128: 505 -> 227 (218 with the chain in the
-// accumulators); with a window of 256 71 -> 50; 2048 rows of 16 heads over 8 of
-// 256: 197 -> 110; 8 rows after 4096 keys, 32 heads over 4: 279 -> 108 (one
-// workgroup a head group: latency).
+// 4096 rows of 32 heads over 8 of 128: 505 -> 221 (218 with the chain in the
+// accumulators); with a window of 256 71 -> 48; 2048 rows of 16 heads over 8 of
+// 256: 197 -> 107; 8 rows after 4096 keys, 32 heads over 4: 279 -> 109 (one
+// workgroup a head group: latency); 8 rows alone, 32 heads over 8: 5.7 -> 6.7 (a
+// tile's 64 keys are copied for 8).
 #include "common.h"
 
 #pragma clang fp contract(off)

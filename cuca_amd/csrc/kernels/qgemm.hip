@@ -186,7 +186,8 @@ __device__ static inline void qgemm_body(const QGemmArgs &a) {
     constexpr int COLS = 64 * RI / (GLU ? 2 : 1); // output columns of a workgroup
     // two buffers of a k-chunk's activations: rows of 256 bytes, 16-byte unit
     // v of row R at unit v ^ (R & 7), so that the reads of 8 rows at one unit
-    // fall in different banks
+    // fall in different banks (rows r and r + 8 of a fragment share theirs: a read
+    // takes 8 cycles, and the LDS pipe is active a quarter of the launch)
     __shared__ __attribute__((aligned(16))) _Float16 xs[2 * TM * QG_KC];
     const int split = SPLIT ? (int)blockIdx.y : 0;
     // XCD x (workgroups x, x + 8, ...) takes row tiles x, x + 8, ... in

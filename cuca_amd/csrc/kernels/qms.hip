@@ -327,8 +327,10 @@ __device__ static inline void qms_body(const QmmArgs &a) {
     }
 }
 
-// Up to 128 registers (four waves a SIMD): 8 waves a workgroup, or (one
-// weight row a lane) up to 16.
+// Up to 128 registers (four waves a SIMD; the four-row Q8_0 kernels use all of
+// them, nothing is spilled): 8 waves a workgroup, or (one weight row a lane) up to
+// 16.  D ring slots: a Q8_0 group is half a Q4_0 group's values, so four slots
+// cover the time of two.
 #define CUCA_QMS(NAME, ...)                                                                \
     extern "C" __global__ __launch_bounds__(8 * CUCA_WAVE, 4) void NAME(QmmArgs a) {        \
         qms_body<__VA_ARGS__>(a);                                                          \

@@ -291,6 +291,7 @@ template <typename T, int FMT, bool UP, int D> __device__ static inline void qms
 #define CUCA_QMS_MOE_SET(TN, T, FN, FMT, D)                        \
     CUCA_QMS_MOE(cuca_qms_moe_up_##TN##_##FN, T, FMT, true, D)     \
     CUCA_QMS_MOE(cuca_qms_moe_down_##TN##_##FN, T, FMT, false, D)
+// (D slots: as qms.hip, but three for Q8_0, down spills with four)
 CUCA_QMS_MOE_SET(f32, float, q4_0, 0, 2)
 CUCA_QMS_MOE_SET(f32, float, q8_0, 1, 3)
 CUCA_QMS_MOE_SET(f16, _Float16, q4_0, 0, 2)
